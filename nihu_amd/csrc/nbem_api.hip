@@ -120,12 +120,32 @@ struct NearList {
 };
 
 struct LaunchCfg {
-	int tile_cols = 32;
+	int tile_cols = 0;      // collocation: 0 = by the size of the grid (regular_tile_cols)
 	int k_batch = 4;
 	int persistent = 4;
 };
 std::mutex g_cfg_mu;
 LaunchCfg g_cfg;
+
+// Trial columns per workgroup of the collocational regular passes.  A lane
+// runs its tile's columns one after another, and a column of near pairs is a
+// long chain of quadrature points, so a small matrix is bound by the chain of
+// one tile: one column per workgroup until the grid holds 16384 workgroups
+// (8 for each of the 2048 that the chip holds at once), then up to 8, which
+// share the row data and the prologue.  Measured, a Burton-Miller call with
+// distance-driven degrees on 300 / 1728 / 8748 / 20172 triangles: 1 column 56
+// / 96 / 789 / 3202 us, 8 columns 83 / 122 / 661 / 2558 us, 32 columns 180 /
+// 229 / 792 / 2671 us; the other passes of the kind alike.  From 2^34 entries
+// on 32 columns keep the grid below 2^32 lanes.
+int regular_tile_cols(int requested, int row_tiles, int n_cols)
+{
+	if (requested > 0) return requested;
+	const long long wg = (long long)row_tiles * n_cols;
+	if (wg >= (1ll << 26)) return 32;
+	int tc = 1;
+	while (tc < 8 && wg / (2 * tc) >= 16384) tc *= 2;
+	return tc;
+}
 
 // per-pass device timing (nb_profile)
 constexpr int NPASS = 4;
@@ -1155,8 +1175,8 @@ int run_quad(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int a
 	std::memset(&a, 0, sizeof(a));
 	a.rmap = jb.rmap; a.cmap = jb.cmap;
 	a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = jb.same;
-	a.tile_cols = jb.tile_cols > 0 ? jb.tile_cols : 32;
 	a.row_tiles = (test->n + 255) / 256;
+	a.tile_cols = regular_tile_cols(jb.tile_cols, a.row_tiles, a.n_cols);
 	a.tn = test->n; a.sn = trial->n;
 	a.tc = (const double *)test->d_c.get();
 	a.tnu = (const float *)test->d_nuf.get();
@@ -1397,8 +1417,8 @@ int run_gauss(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int 
 	nbk::GaussArgs a;
 	std::memset(&a, 0, sizeof(a));
 	a.n_rows = nodes * test->n; a.n_cols = trial->n; a.same_mesh = jb.same; a.nodes = nodes;
-	a.tile_cols = jb.tile_cols > 0 ? jb.tile_cols : 32;
 	a.row_tiles = (a.n_rows + 255) / 256;
+	a.tile_cols = regular_tile_cols(jb.tile_cols, a.row_tiles, a.n_cols);
 	a.tn = a.n_rows; a.te = test->n;
 	a.tx = (const double *)(tg ? test->d_gx.get() : test->d_c.get());
 	a.tnu = (const float *)(tg ? test->d_gnuf.get() : test->d_nuf.get());
@@ -1577,8 +1597,8 @@ int run_device(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int
 	std::memset(&a, 0, sizeof(a));
 	a.rmap = jb.rmap; a.cmap = jb.cmap;
 	a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = jb.same;
-	a.tile_cols = jb.tile_cols > 0 ? jb.tile_cols : 32;
 	a.row_tiles = (test->n + 255) / 256;
+	a.tile_cols = regular_tile_cols(jb.tile_cols, a.row_tiles, a.n_cols);
 	a.tn = test->n; a.sn = trial->n;
 	a.tc = (const double *)test->d_c.get();
 	a.tnu = (const float *)test->d_nuf.get();
@@ -1996,7 +2016,7 @@ int sweep_impl(const nb_mesh *mesh, const double *k, int32_t n_k, const nb_polic
 			Job jb;
 			jb.test = m; jb.trial = m; jb.formalism = NB_COLLOCATION; jb.same = 1; jb.family = NB_HELMHOLTZ;
 			jb.km = nbk::ALL4; jb.mode = nbk::OUT_BM;
-			jb.k = k[f]; jb.alpha = {0.0, -1.0 / k[f]}; jb.pol = *policy; jb.tile_cols = 32;
+			jb.k = k[f]; jb.alpha = {0.0, -1.0 / k[f]}; jb.pol = *policy; jb.tile_cols = 0;
 			if ((s = run_any(jb, (float2 *)A + f * k_stride, (float2 *)B + f * k_stride, ld, NB_C64, 0, st))) return s;
 		}
 		return NB_OK;

@@ -1,0 +1,75 @@
+"""Sizes at which the launch shapes change or leave remainders: element counts
+around a wave, a workgroup and the steps of the trial-column rule, compared
+with the FP64 oracle on sampled rows (the first, the last and those at the
+edges of a workgroup's 256 rows), every column.
+
+Bars as in the parity tests: 2e-6 of the row's largest entry and 1e-5 relative
+Frobenius (FP32 regular pairs)."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+NIHU = (dict(rule="nihu", near="mean_edge", limit=1.5), dict(rule=0, fixed_degree=0, near_mode=0, near_limit=1.5))
+SEVEN = (dict(rule="fixed", degree=5, near="diameter", limit=2.0),
+         dict(rule=1, fixed_degree=5, near_mode=1, near_limit=2.0))
+
+
+@pytest.fixture(scope="module")
+def nb():
+    import torch
+    assert torch.cuda.is_available(), "GPU test without a GPU"
+    from nihu_amd import nbem
+    return nbem
+
+
+def check(got, ref):
+    scale = np.abs(ref).max(axis=1, keepdims=True)
+    assert (np.abs(got - ref) / scale).max() < 2e-6
+    assert np.linalg.norm(got - ref) < 1e-5 * np.linalg.norm(ref)
+
+
+def surface(n_elem, quads=False):
+    """the first n_elem elements of a cube sphere (triangles: its squares cut in two, jittered)"""
+    from nihu_amd.mesh import cubed_sphere
+    n = int(np.ceil(np.sqrt(n_elem / (6 if quads else 12))))
+    nodes, q = cubed_sphere(n)
+    if quads:
+        return nodes, np.ascontiguousarray(q[:n_elem])
+    nodes = nodes * (1.0 + np.random.default_rng(n_elem).uniform(-0.01, 0.01, len(nodes)))[:, None]
+    t = np.concatenate([q[:, None, [0, 1, 2]], q[:, None, [0, 2, 3]]], axis=1).reshape(-1, 3)
+    return nodes, np.ascontiguousarray(t[:n_elem])
+
+
+def sample(n):
+    return np.unique([r for r in (0, 63, 64, 255, 256, 511, 512, n - 2, n - 1) if 0 <= r < n]).astype(np.int32)
+
+
+@pytest.mark.parametrize("policy", [NIHU, SEVEN], ids=["nihu", "seven"])
+@pytest.mark.parametrize("n_elem", [1, 63, 65, 255, 257, 1999, 3001, 5003, 9001])
+def test_burton_miller_triangles(nb, orc, n_elem, policy):
+    import torch
+    nodes, tris = surface(n_elem)
+    m = nb.Mesh(nodes, tris)
+    A, B = nb.colmajor(n_elem, n_elem), nb.colmajor(n_elem, n_elem)
+    nb.assemble_bm(m, 4.0, A, B, pol=nb.policy(**policy[0]))
+    torch.cuda.synchronize()
+    rows = sample(n_elem)
+    Ar, Br = orc.assemble_bm(nodes, tris, 4.0, pol=orc.policy(**policy[1]), rows=rows)
+    check(A[rows].cpu().numpy(), Ar)
+    check(B[rows].cpu().numpy(), Br)
+
+
+@pytest.mark.parametrize("n_elem", [1, 63, 65, 257, 2999, 9001])
+def test_burton_miller_quadrilaterals(nb, orc, n_elem):
+    import torch
+    nodes, quads = surface(n_elem, quads=True)
+    m = nb.Mesh(nodes, quads)
+    A, B = nb.colmajor(n_elem, n_elem), nb.colmajor(n_elem, n_elem)
+    nb.assemble_bm(m, 4.0, A, B)
+    torch.cuda.synchronize()
+    rows = sample(n_elem)
+    Ar, Br = orc.assemble_bm(nodes, quads, 4.0, rows=rows)
+    check(A[rows].cpu().numpy(), Ar)
+    check(B[rows].cpu().numpy(), Br)
