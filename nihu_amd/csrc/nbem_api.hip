@@ -147,6 +147,21 @@ int regular_tile_cols(int requested, int row_tiles, int n_cols)
 	return tc;
 }
 
+// log2 of the lanes per pair of an FP64 pass (near-singular, diagonal): from
+// `least`, doubled up to `most` while the launch has fewer than 2^16 lanes (a
+// wave for each of the chip's 1024 SIMDs): below that the time is one pair's
+// chain of points, above it their issue, to which every further lane adds its
+// setup.  Near pass of 864 quadrilaterals with 2^16 / 2^17 / 2^18 / 2^19 lanes
+// 67 / 83 / 84 / 83 us, of 1944 105 / 117 / 171 / 172, of 1728 triangles 31 /
+// 33 / 47 / 81 (4 lanes a quadrilateral pair and 1 a triangle pair: 100-140
+// and 60 us whatever the size).
+int fp64_lanes_log2(long long pairs, int least, int most)
+{
+	int l = least;
+	while (l < most && (pairs << l) < (1ll << 16)) ++l;
+	return l;
+}
+
 // per-pass device timing (nb_profile)
 constexpr int NPASS = 4;
 std::mutex g_prof_mu;
@@ -1320,8 +1335,9 @@ int run_quad(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int a
 		na.pi = diag ? nullptr : (const int *)nl->pi.get();
 		na.pj = diag ? nullptr : (const int *)nl->pj.get();
 		if (na.n_pairs == 0) continue;
-		// diagonal: one lane per element; near: QLPP lanes per pair
-		const long long lanes = (long long)na.n_pairs * (diag ? 1 : nbk::QLPP);
+		// near: 4 lanes per pair and more for short lists; diagonal: 8 to 32
+		na.lpp_log2 = fp64_lanes_log2(na.n_pairs, diag ? 3 : 2, 5);
+		const long long lanes = (long long)na.n_pairs << na.lpp_log2;
 		const int g = (int)((lanes + 63) / 64);
 		const int pe = prof_begin(diag ? 2 : 1, side);
 		using namespace nbk;
@@ -1534,8 +1550,9 @@ int run_gauss(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int 
 		na.pi = diag ? nullptr : (const int *)nl->pi.get();
 		na.pj = diag ? nullptr : (const int *)nl->pj.get();
 		if (na.n_pairs == 0) continue;
-		// diagonal: one lane per (element, node); near: QLPP lanes per (pair, node)
-		const long long lanes = (long long)na.n_pairs * nodes * (diag ? 1 : nbk::QLPP);
+		// near: 4 lanes per (pair, node) and more for short lists; diagonal: 8 to 32
+		na.lpp_log2 = fp64_lanes_log2((long long)na.n_pairs * nodes, diag ? 3 : 2, 5);
+		const long long lanes = ((long long)na.n_pairs * nodes) << na.lpp_log2;
 		const int g = (int)((lanes + 63) / 64);
 		const int pe = prof_begin(diag ? 2 : 1, st);
 		using namespace nbk;
@@ -1731,7 +1748,8 @@ int run_device(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int
 		na.pi = diag ? nullptr : (const int *)nl->pi.get();
 		na.pj = diag ? nullptr : (const int *)nl->pj.get();
 		if (na.n_pairs == 0) continue;
-		const int g = (na.n_pairs + 63) / 64;
+		na.lpp_log2 = fp64_lanes_log2(na.n_pairs, 0, diag ? 4 : 5);
+		const int g = (int)((((long long)na.n_pairs << na.lpp_log2) + 63) / 64);
 		const int pe = prof_begin(diag ? 2 : 1, side);
 		using namespace nbk;
 #define NB_FP64(F, K, M) do { \

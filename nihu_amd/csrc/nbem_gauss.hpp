@@ -19,12 +19,12 @@
 //   near (FP64, d / R < 1.5 between centres): per test node the polar method
 //     with F = K J N(xi) - K_lin J_lin N(xi0) and the planar integral times
 //     N(xi0) (nearly_singular_collocational.hpp:86-197), or Telles with N(xi)
-//     in the weights; QLPP lanes per (pair, node);
+//     in the weights; 4 lanes per (pair, node) or more;
 //   singular (FP64, the same element): per node xi_a the order-7 Duffy blind
 //     rule around xi_a, and Guiggiani's method at xi_a for HSP with the
 //     shape-function terms of the Laurent coefficients, a0 N_b(xi_a) and
 //     a1 N_b(xi_a) + a0 grad N_b(xi_a).v (guiggiani_1992.hpp:180-330,
-//     laplace_kernel.hpp:266-295); one lane per (element, node).
+//     laplace_kernel.hpp:266-295); 8 lanes per (element, node) or more.
 
 #pragma once
 
@@ -316,6 +316,7 @@ struct GaussNearArgs {
 	const Rules *rules;
 	int *status;                 // pairs without an inverse image (null: none kept)
 	int inv_iter;
+	int lpp_log2;                // log2 of the lanes that share one (pair, node)
 };
 
 // the shape functions at (xi, eta), and the nodes
@@ -361,10 +362,10 @@ __device__ __forceinline__ void gspread(const double (&N)[GDOF], const double2 (
 template <int FAM, int MASK, bool CK>
 __device__ bool gauss_near_polar(const Quad &Q, D3 x0, D3 nx0, double k, int nr, const double *grx, const double *grw,
 	int nt, const double *gtx, const double *gtw, const Rules &R, double2 (&s)[GDOF][4], int lane, int nl,
-	int max_iter, double ki)
+	int max_iter, InverseMap &im, double ki)
 {
-	double xi0, eta0, zeta;
-	if (!quad_inverse(Q, x0, 1e-5, max_iter, xi0, eta0, zeta)) return false;
+	if (!quad_inverse(Q, x0, 1e-5, max_iter, im)) return false;
+	const double xi0 = im.xi, eta0 = im.eta;
 	D3 a, b;
 	quad_dx(Q, xi0, eta0, a, b);
 	const D3 xl0 = quad_x(Q, xi0, eta0);
@@ -396,7 +397,7 @@ __device__ bool gauss_near_polar(const Quad &Q, D3 x0, D3 nx0, double k, int nr,
 			else t2 += 2.0 * PI_D;
 		}
 		if (fabs(t2 - t1) < 1e-3) continue;
-		for (int it = (lane + nt * nl - (nt * n) % nl) % nl; it < nt; it += nl) {
+		for (int it = (lane - nt * n) & (nl - 1); it < nt; it += nl) {
 			const double th = ((1.0 - gtx[it]) * t1 + (1.0 + gtx[it]) * t2) / 2.0;
 			const double wt = gtw[it] * (t2 - t1) / 2.0;
 			double st, ct;
@@ -436,10 +437,10 @@ __device__ bool gauss_near_polar(const Quad &Q, D3 x0, D3 nx0, double k, int nr,
 // Telles-transformed order-30 rule with the shape functions (quad_near_telles)
 template <int FAM, int MASK, bool CK>
 __device__ bool gauss_near_telles(const Quad &Q, D3 x0, D3 nx0, double k, const Rules &R, double2 (&s)[GDOF][4],
-	int lane, int nl, int max_iter, double ki)
+	int lane, int nl, int max_iter, InverseMap &im, double ki)
 {
-	double xi0, eta0, zeta;
-	if (!quad_inverse(Q, x0, 1e-6, max_iter, xi0, eta0, zeta)) return false;
+	if (!quad_inverse(Q, x0, 1e-6, max_iter, im)) return false;
+	const double xi0 = im.xi, eta0 = im.eta, zeta = im.zeta;
 	double rb;
 	if (zeta < 0.05) rb = 0.0;
 	else if (zeta <= 1.3) rb = 0.85 + 0.24 * log(zeta);
@@ -448,11 +449,13 @@ __device__ bool gauss_near_telles(const Quad &Q, D3 x0, D3 nx0, double k, const 
 	double a0, b0, c0, e0, a1, b1, c1, e1;
 	telles_coeffs(xi0, rb, a0, b0, c0, e0);
 	telles_coeffs(eta0, rb, a1, b1, c1, e1);
-	for (int i = lane; i < 16; i += nl) {
+	// up to 16 lanes take whole lines, more share the points of each
+	const int nj = nl > 16 ? nl >> 4 : 1;
+	for (int i = lane & 15; i < 16; i += nl) {
 		const double x = R.gl16x[i];
 		const double xi = a0 * x * x * x + b0 * x * x + c0 * x + e0;
 		const double jx = 3.0 * a0 * x * x + 2.0 * b0 * x + c0;
-		for (int j = 0; j < 16; ++j) {
+		for (int j = lane >> 4; j < 16; j += nj) {
 			const double y = R.gl16x[j];
 			const double eta = a1 * y * y * y + b1 * y * y + c1 * y + e1;
 			const double jy = 3.0 * a1 * y * y + 2.0 * b1 * y + c1;
@@ -472,7 +475,7 @@ __device__ bool gauss_near_telles(const Quad &Q, D3 x0, D3 nx0, double k, const 
 // a1 N_b(xi0) + a0 grad N_b(xi0).v, v the direction in the reference square).
 template <int FAM, bool CK>
 __device__ void gauss_guiggiani(const Quad &Q, double xi0x, double xi0y, double k, const Rules &R, double ki,
-	double2 (&s)[GDOF][4])
+	double2 (&s)[GDOF][4], int lane, int nl)
 {
 	D3 dxi, deta;
 	quad_dx(Q, xi0x, xi0y, dxi, deta);
@@ -513,7 +516,7 @@ __device__ void gauss_guiggiani(const Quad &Q, double xi0x, double xi0y, double 
 		double t2 = th_lim[n == 3 ? 0 : n + 1];
 		if (fabs(t2 - t1) < 1e-3) continue;
 		if (fabs(t2 - t1) > PI_D) t2 += 2.0 * PI_D;
-		for (int it = 0; it < 5; ++it) {
+		for (int it = (lane - 5 * n) & (nl - 1); it < 5; it += nl) {
 			const double th = ((1.0 - R.gl5x[it]) * t1 + (1.0 + R.gl5x[it]) * t2) / 2.0;
 			const double wt = R.gl5w[it] * (t2 - t1) / 2.0;
 			double st, ct;
@@ -689,13 +692,26 @@ __device__ __forceinline__ void gauss_load(const GaussNearArgs &a, int row, int 
 	nx = {a.tnu[row], a.tnu[a.tn + row], a.tnu[2 * a.tn + row]};
 }
 
-// Diagonal blocks: one lane per (element, node): Duffy around the node for
-// SLP / DLP / DLPt, Guiggiani there for HSP.
+// the sums of a (pair, node) over its nl lanes
+template <int KM>
+__device__ __forceinline__ void gauss_lane_sum(double2 (&s)[GDOF][4], int nl)
+{
+#pragma unroll
+	for (int d = 0; d < GDOF; ++d)
+#pragma unroll
+		for (int t = 0; t < 4; ++t)
+			if (KM & (1 << t)) s[d][t] = pair_sum(s[d][t], nl);
+}
+
+// Diagonal blocks: 2^lpp_log2 lanes per (element, node): Duffy around the node
+// for SLP / DLP / DLPt, Guiggiani there for HSP.
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(64) gauss_diag_kernel(GaussNearArgs a)
 {
 	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-	const int e = gid >> 2, node = gid & 3;
+	const int nl = 1 << a.lpp_log2, lane = gid & (nl - 1);
+	const int en = gid >> a.lpp_log2;
+	const int e = en >> 2, node = en & 3;
 	if (e >= a.n_pairs) return;
 	const Rules &R = *a.rules;
 	const int row = GDOF * e + node;
@@ -707,7 +723,7 @@ __global__ void __launch_bounds__(64) gauss_diag_kernel(GaussNearArgs a)
 		for (int t = 0; t < 4; ++t) s[d][t] = make_double2(0, 0);
 	constexpr int WEAK = KM & (SLP | DLP | DLPT);
 	if (WEAK)
-		for (int q = 0; q < 64; ++q) {
+		for (int q = lane; q < 64; q += nl) {
 			const double xi = R.gduffy[node][q][0], eta = R.gduffy[node][q][1];
 			double2 f[4] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
 			quad_kernel_at<FAM, WEAK, CK>(Q, xi, eta, x0, nx, a.k, R.gduffy[node][q][2], f, a.ki);
@@ -718,19 +734,21 @@ __global__ void __launch_bounds__(64) gauss_diag_kernel(GaussNearArgs a)
 	if (KM & HSP) {
 		double xi0, eta0;
 		gnode64(node, xi0, eta0);
-		gauss_guiggiani<FAM, CK>(Q, xi0, eta0, a.k, R, a.ki, s);
+		gauss_guiggiani<FAM, CK>(Q, xi0, eta0, a.k, R, a.ki, s, lane, nl);
 	}
-	gauss_store64<KM, MODE, true>(a, row, e, node, s);
+	gauss_lane_sum<KM>(s, nl);
+	if (lane == 0) gauss_store64<KM, MODE, true>(a, row, e, node, s);
 }
 
-// Near-singular pairs: QLPP lanes per (pair, test node), then a butterfly sum
-// over the lanes; the first lane stores the node's four dofs.
+// Near-singular pairs: 2^lpp_log2 lanes (4 or more) per (pair, test node),
+// then a butterfly sum over the lanes; the first lane stores the node's four
+// dofs.
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(64) gauss_near_kernel(GaussNearArgs a)
 {
 	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-	const int lane = gid % QLPP;
-	const int pn = gid / QLPP;
+	const int nl = 1 << a.lpp_log2, lane = gid & (nl - 1);
+	const int pn = gid >> a.lpp_log2;
 	const int p = pn / a.nodes, node = pn % a.nodes;
 	// lanes past the last pair repeat it and do not store
 	const bool valid = p < a.n_pairs;
@@ -745,26 +763,22 @@ __global__ void __launch_bounds__(64) gauss_near_kernel(GaussNearArgs a)
 	for (int d = 0; d < GDOF; ++d)
 		for (int t = 0; t < 4; ++t) s[d][t] = make_double2(0, 0);
 	bool ok = true;
+	InverseMap im;
 	if (FAM == HELM) {
 		if (KM & SLP)
-			ok = gauss_near_polar<FAM, SLP, CK>(Q, x0, nx, a.k, 8, R.gl8x, R.gl8w, 8, R.gl8x, R.gl8w, R, s, lane, QLPP,
-				a.inv_iter, a.ki);
+			ok = gauss_near_polar<FAM, SLP, CK>(Q, x0, nx, a.k, 8, R.gl8x, R.gl8w, 8, R.gl8x, R.gl8w, R, s, lane, nl,
+				a.inv_iter, im, a.ki);
 		if (ok && (KM & (DLP | DLPT | HSP)))
-			ok = gauss_near_telles<FAM, KM & (DLP | DLPT | HSP), CK>(Q, x0, nx, a.k, R, s, lane, QLPP, a.inv_iter, a.ki);
+			ok = gauss_near_telles<FAM, KM & (DLP | DLPT | HSP), CK>(Q, x0, nx, a.k, R, s, lane, nl, a.inv_iter, im, a.ki);
 	} else {
 		if (KM & (SLP | DLP | DLPT))
 			ok = gauss_near_polar<FAM, KM & (SLP | DLP | DLPT), false>(Q, x0, nx, 0.0, 8, R.gl8x, R.gl8w, 8, R.gl8x,
-				R.gl8w, R, s, lane, QLPP, a.inv_iter, 0.0);
+				R.gl8w, R, s, lane, nl, a.inv_iter, im, 0.0);
 		if (ok && (KM & HSP))
 			ok = gauss_near_polar<FAM, HSP, false>(Q, x0, nx, 0.0, 51, R.gl51x, R.gl51w, 51, R.gl51x, R.gl51w, R, s,
-				lane, QLPP, a.inv_iter, 0.0);
+				lane, nl, a.inv_iter, im, 0.0);
 	}
-	for (int off = QLPP / 2; off >= 1; off >>= 1)
-		for (int d = 0; d < GDOF; ++d)
-			for (int t = 0; t < 4; ++t) {
-				s[d][t].x += __shfl_xor(s[d][t].x, off, QLPP);
-				s[d][t].y += __shfl_xor(s[d][t].y, off, QLPP);
-			}
+	gauss_lane_sum<KM>(s, nl);
 	if (!ok) {
 		const double nan = __builtin_nan("");
 		for (int d = 0; d < GDOF; ++d)

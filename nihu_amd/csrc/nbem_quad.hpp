@@ -20,12 +20,12 @@
 // and n_x.n_y are per point.  The one-point rule (every far pair) is the
 // centre with weight 4 J(0, 0): no table load, FP64-reduced phase.
 // FP64 pass:
-//   diagonal (one lane per element): SLP / DLP / DLPt by the order-7 Duffy blind rule around the
+//   diagonal (8 lanes per element or more): SLP / DLP / DLPt by the order-7 Duffy blind rule around the
 //     centre (nihu/core/singular_accelerator.hpp:363-456,
 //     nihu/core/duffy_quadrature.hpp); HSP by Guiggiani's method with orders
 //     (5, 9) (nihu/library/guiggiani_1992.hpp:138-330, Laurent coefficients
 //     of the Laplace HSP core nihu/library/laplace_kernel.hpp:266-295);
-//   near (d / R < limit; 4 lanes per pair): Helmholtz SLP and Laplace SLP / DLP / DLPt by polar
+//   near (d / R < limit; 4 lanes per pair or more): Helmholtz SLP and Laplace SLP / DLP / DLPt by polar
 //     integration around the image of x0 of K J - K_lin J_lin plus the planar
 //     integral over the linearised element (orders 15 x 15; Laplace HSP
 //     100 x 100) (nihu/library/nearly_singular_collocational.hpp:71-203);
@@ -429,9 +429,10 @@ __device__ __forceinline__ void quad_kernel_at(const Quad &Q, double xi, double 
 
 // Singular SLP / DLP / DLPt: the order-7 Duffy rule around the centre
 template <int FAM, int MASK, bool CK = false>
-__device__ void quad_blind(const Quad &Q, D3 x0, D3 nx0, double k, const Rules &R, double2 (&s)[4], double ki = 0.0)
+__device__ void quad_blind(const Quad &Q, D3 x0, D3 nx0, double k, const Rules &R, double2 (&s)[4], double ki, int lane,
+	int nl)
 {
-	for (int q = 0; q < 64; ++q)
+	for (int q = lane; q < 64; q += nl)
 		quad_kernel_at<FAM, MASK, CK>(Q, R.duffy[q][0], R.duffy[q][1], x0, nx0, k, R.duffy[q][2], s, ki);
 }
 
@@ -440,7 +441,7 @@ __device__ void quad_blind(const Quad &Q, D3 x0, D3 nx0, double k, const Rules &
 // normal there.  A complex wavenumber (CK) leaves the Laurent terms as they
 // are: it enters the HSP kernel first at order 1 / r, bounded under rho.
 template <int FAM, bool CK = false>
-__device__ double2 quad_guiggiani(const Quad &Q, double k, const Rules &R, double ki = 0.0)
+__device__ double2 quad_guiggiani(const Quad &Q, double k, const Rules &R, double ki, int lane, int nl)
 {
 	D3 dxi, deta;
 	quad_dx(Q, 0.0, 0.0, dxi, deta);
@@ -478,7 +479,7 @@ __device__ double2 quad_guiggiani(const Quad &Q, double k, const Rules &R, doubl
 		double t2 = th_lim[n == 3 ? 0 : n + 1];
 		if (fabs(t2 - t1) < 1e-3) continue;
 		if (fabs(t2 - t1) > PI_D) t2 += 2.0 * PI_D;
-		for (int it = 0; it < 5; ++it) {
+		for (int it = (lane - 5 * n) & (nl - 1); it < 5; it += nl) {
 			const double th = ((1.0 - R.gl5x[it]) * t1 + (1.0 + R.gl5x[it]) * t2) / 2.0;
 			const double wt = R.gl5w[it] * (t2 - t1) / 2.0;
 			double st, ct;
@@ -518,19 +519,23 @@ __device__ double2 quad_guiggiani(const Quad &Q, double k, const Rules &R, doubl
 
 // Image (xi, eta) and normal offset zeta of x0: x(xi) + zeta n / sqrt|n| = x0
 // by Newton-Raphson from 0 (at most max_iter steps -- NiHu's 100 -- with
-// |residual| < tol).
-__device__ bool quad_inverse(const Quad &Q, D3 x0, double tol, int max_iter, double &xi, double &eta, double &zeta)
+// |residual| < tol).  The iteration starts from the state in `m` and leaves
+// it there, so that a second search to a smaller tolerance goes on where the
+// first one stopped (the iterates are those of a search from 0).
+struct InverseMap { double xi = 0.0, eta = 0.0, zeta = 0.0; int it = 0; };
+
+__device__ bool quad_inverse(const Quad &Q, D3 x0, double tol, int max_iter, InverseMap &m)
 {
-	double r0 = 0.0, r1 = 0.0, r2 = 0.0;
+	double r0 = m.xi, r1 = m.eta, r2 = m.zeta;
 	const D3 dxe = quad_dxe(Q);
-	for (int it = 0; it < max_iter; ++it) {
+	for (int it = m.it; it < max_iter; ++it) {
 		D3 a, b;
 		quad_dx(Q, r0, r1, a, b);
 		D3 n = d3cross(a, b);
 		const double sj = sqrt(d3norm(n));
 		n = d3scale(n, 1.0 / sj);
 		const D3 f = d3sub(d3add(quad_x(Q, r0, r1), d3scale(n, r2)), x0);
-		if (d3norm(f) < tol) { xi = r0; eta = r1; zeta = r2; return true; }
+		if (d3norm(f) < tol) { m.xi = r0; m.eta = r1; m.zeta = r2; m.it = it; return true; }
 		const D3 c0 = d3add(a, d3scale(d3cross(a, dxe), r2 / sj));
 		const D3 c1 = d3add(b, d3scale(d3cross(dxe, b), r2 / sj));
 		// solve [c0 c1 n] d = f by Gaussian elimination with partial pivoting
@@ -562,10 +567,10 @@ __device__ bool quad_inverse(const Quad &Q, D3 x0, double tol, int max_iter, dou
 template <int FAM, int MASK, bool CK = false>
 __device__ bool quad_near_polar(const Quad &Q, D3 x0, D3 nx0, double k, int nr, const double *grx, const double *grw,
 	int nt, const double *gtx, const double *gtw, const Rules &R, double2 (&s)[4], int lane, int nl, int max_iter,
-	double ki = 0.0)
+	InverseMap &im, double ki = 0.0)
 {
-	double xi0, eta0, zeta;
-	if (!quad_inverse(Q, x0, 1e-5, max_iter, xi0, eta0, zeta)) return false;
+	if (!quad_inverse(Q, x0, 1e-5, max_iter, im)) return false;
+	const double xi0 = im.xi, eta0 = im.eta;
 	// the tangent parallelogram at xi0: x_lin(xi) = xl0 + a (xi - xi0) + b (eta - eta0)
 	D3 a, b;
 	quad_dx(Q, xi0, eta0, a, b);
@@ -596,7 +601,7 @@ __device__ bool quad_near_polar(const Quad &Q, D3 x0, D3 nx0, double k, int nr, 
 			else t2 += 2.0 * PI_D;
 		}
 		if (fabs(t2 - t1) < 1e-3) continue;
-		for (int it = (lane + nt * nl - (nt * n) % nl) % nl; it < nt; it += nl) {
+		for (int it = (lane - nt * n) & (nl - 1); it < nt; it += nl) {
 			const double th = ((1.0 - gtx[it]) * t1 + (1.0 + gtx[it]) * t2) / 2.0;
 			const double wt = gtw[it] * (t2 - t1) / 2.0;
 			double st, ct;
@@ -644,10 +649,10 @@ __device__ __forceinline__ void telles_coeffs(double e, double rb, double &ca, d
 
 template <int FAM, int MASK, bool CK = false>
 __device__ bool quad_near_telles(const Quad &Q, D3 x0, D3 nx0, double k, const Rules &R, double2 (&s)[4], int lane,
-	int nl, int max_iter, double ki = 0.0)
+	int nl, int max_iter, InverseMap &im, double ki = 0.0)
 {
-	double xi0, eta0, zeta;
-	if (!quad_inverse(Q, x0, 1e-6, max_iter, xi0, eta0, zeta)) return false;
+	if (!quad_inverse(Q, x0, 1e-6, max_iter, im)) return false;
+	const double xi0 = im.xi, eta0 = im.eta, zeta = im.zeta;
 	double rb;
 	if (zeta < 0.05) rb = 0.0;
 	else if (zeta <= 1.3) rb = 0.85 + 0.24 * log(zeta);
@@ -656,11 +661,13 @@ __device__ bool quad_near_telles(const Quad &Q, D3 x0, D3 nx0, double k, const R
 	double a0, b0, c0, e0, a1, b1, c1, e1;
 	telles_coeffs(xi0, rb, a0, b0, c0, e0);
 	telles_coeffs(eta0, rb, a1, b1, c1, e1);
-	for (int i = lane; i < 16; i += nl) {
+	// up to 16 lanes take whole lines, more share the points of each
+	const int nj = nl > 16 ? nl >> 4 : 1;
+	for (int i = lane & 15; i < 16; i += nl) {
 		const double x = R.gl16x[i];
 		const double xi = a0 * x * x * x + b0 * x * x + c0 * x + e0;
 		const double jx = 3.0 * a0 * x * x + 2.0 * b0 * x + c0;
-		for (int j = 0; j < 16; ++j) {
+		for (int j = lane >> 4; j < 16; j += nj) {
 			const double y = R.gl16x[j];
 			const double eta = a1 * y * y * y + b1 * y * y + c1 * y + e1;
 			const double jy = 3.0 * a1 * y * y + 2.0 * b1 * y + c1;
@@ -785,32 +792,37 @@ __device__ __forceinline__ void quad_load(const NearArgs &a, int i, int j, Quad 
 	nx = {a.tnu[i], a.tnu[a.tn + i], a.tnu[2 * a.tn + i]};
 }
 
-// Diagonal pairs: one lane per element (Duffy rule, Guiggiani).
+// Diagonal pairs (Duffy rule, Guiggiani): 2^lpp_log2 lanes per element share
+// the 64 points and the 20 angular lines.
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(64) quad_diag_kernel(NearArgs a)
 {
-	const int p = blockIdx.x * blockDim.x + threadIdx.x;
+	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+	const int nl = 1 << a.lpp_log2, lane = gid & (nl - 1);
+	const int p = gid >> a.lpp_log2;
 	if (p >= a.n_pairs) return;
 	const Rules &R = *a.rules;
 	Quad Q;
 	D3 x0, nx;
 	quad_load(a, p, p, Q, x0, nx);
 	double2 s[4] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
-	if (KM & (SLP | DLP | DLPT)) quad_blind<FAM, KM & (SLP | DLP | DLPT), CK>(Q, x0, nx, a.k, R, s, a.ki);
-	if (KM & HSP) s[3] = quad_guiggiani<FAM, CK>(Q, a.k, R, a.ki);
-	quad_store64<KM, MODE, true>(a, p, p, s);
+	if (KM & (SLP | DLP | DLPT)) quad_blind<FAM, KM & (SLP | DLP | DLPT), CK>(Q, x0, nx, a.k, R, s, a.ki, lane, nl);
+	if (KM & HSP) s[3] = quad_guiggiani<FAM, CK>(Q, a.k, R, a.ki, lane, nl);
+	for (int t = 0; t < 4; ++t)
+		if (KM & (1 << t)) s[t] = pair_sum(s[t], nl);
+	if (lane == 0) quad_store64<KM, MODE, true>(a, p, p, s);
 }
 
-// Near-singular pairs: QLPP lanes per pair share the angular lines, planar
-// and Telles points (each lane repeats the pair's inverse mapping), then a
-// butterfly sum over the lanes; the pair's first lane stores.
-constexpr int QLPP = 4;
-
+// Near-singular pairs: 2^lpp_log2 lanes per pair (4 or more) share the
+// angular lines, planar and Telles points (each lane repeats the pair's
+// inverse mapping), then a butterfly sum over the lanes; the pair's first
+// lane stores.
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(64, 3) quad_near_kernel(NearArgs a)
 {
 	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-	const int p = gid / QLPP, lane = gid % QLPP;
+	const int nl = 1 << a.lpp_log2, lane = gid & (nl - 1);
+	const int p = gid >> a.lpp_log2;
 	// lanes past the last pair repeat it and do not store
 	const bool valid = p < a.n_pairs;
 	const int pp = valid ? p : a.n_pairs - 1;
@@ -821,26 +833,24 @@ __global__ void __launch_bounds__(64, 3) quad_near_kernel(NearArgs a)
 	quad_load(a, i, j, Q, x0, nx);
 	double2 s[4] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
 	bool ok = true;
+	InverseMap im;
 	if (FAM == HELM) {
 		if (KM & SLP)
-			ok = quad_near_polar<FAM, SLP, CK>(Q, x0, nx, a.k, 8, R.gl8x, R.gl8w, 8, R.gl8x, R.gl8w, R, s, lane, QLPP,
-				a.inv_iter, a.ki);
+			ok = quad_near_polar<FAM, SLP, CK>(Q, x0, nx, a.k, 8, R.gl8x, R.gl8w, 8, R.gl8x, R.gl8w, R, s, lane, nl,
+				a.inv_iter, im, a.ki);
 		if (ok && (KM & (DLP | DLPT | HSP)))
-			ok = quad_near_telles<FAM, KM & (DLP | DLPT | HSP), CK>(Q, x0, nx, a.k, R, s, lane, QLPP, a.inv_iter,
+			ok = quad_near_telles<FAM, KM & (DLP | DLPT | HSP), CK>(Q, x0, nx, a.k, R, s, lane, nl, a.inv_iter, im,
 				a.ki);
 	} else {
 		if (KM & (SLP | DLP | DLPT))
 			ok = quad_near_polar<FAM, KM & (SLP | DLP | DLPT)>(Q, x0, nx, 0.0, 8, R.gl8x, R.gl8w, 8, R.gl8x, R.gl8w, R, s,
-				lane, QLPP, a.inv_iter);
+				lane, nl, a.inv_iter, im);
 		if (ok && (KM & HSP))
-			ok = quad_near_polar<FAM, HSP>(Q, x0, nx, 0.0, 51, R.gl51x, R.gl51w, 51, R.gl51x, R.gl51w, R, s, lane, QLPP,
-				a.inv_iter);
+			ok = quad_near_polar<FAM, HSP>(Q, x0, nx, 0.0, 51, R.gl51x, R.gl51w, 51, R.gl51x, R.gl51w, R, s, lane, nl,
+				a.inv_iter, im);
 	}
-	for (int off = QLPP / 2; off >= 1; off >>= 1)
-		for (int t = 0; t < 4; ++t) {
-			s[t].x += __shfl_xor(s[t].x, off, QLPP);
-			s[t].y += __shfl_xor(s[t].y, off, QLPP);
-		}
+	for (int t = 0; t < 4; ++t)
+		if (KM & (1 << t)) s[t] = pair_sum(s[t], nl);
 	if (!ok) {
 		// the inverse mapping did not converge (NiHu throws): NaN marks the
 		// entry and the pair is counted, so that the call reports an error
