@@ -564,7 +564,7 @@ void policy_degrees(const nb_policy &p, int km, int field_complexity, std::vecto
 	deg.erase(std::unique(deg.begin(), deg.end()), deg.end());
 }
 
-// the cached near-pair list of (test mesh, near policy), or null
+// the cached list of (test mesh, near policy), or null
 std::shared_ptr<NearList> find_near_list(const nb_mesh *trial, const nb_mesh *test, int same, const nb_policy &pol)
 {
 	for (auto &nl : trial->near_cache)
@@ -573,9 +573,18 @@ std::shared_ptr<NearList> find_near_list(const nb_mesh *trial, const nb_mesh *te
 	return nullptr;
 }
 
-int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, const nb_policy &pol, hipStream_t st,
-	std::shared_ptr<NearList> *out)
+// Near-pair lists.  slot THR_NEAR: the near-singular pairs of a policy.
+// Another slot: the pairs of the Galerkin formalism inside that breakpoint of
+// the distance tables that share no node (kept under the mode GAL_LIST + slot).
+constexpr int GAL_LIST = 64;
+
+int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy pol, hipStream_t st,
+	std::shared_ptr<NearList> *out, int slot = nbk::THR_NEAR)
 {
+	if (slot != nbk::THR_NEAR) {
+		pol.near_mode = GAL_LIST + slot;
+		pol.near_limit = 0.0;
+	}
 	if ((*out = find_near_list(trial, test, same, pol))) return NB_OK;
 	std::shared_ptr<NearList> nl(new NearList());
 	nl->test_uid = test->uid; nl->same = same; nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0;
@@ -588,7 +597,11 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, const nb_pol
 		a.tn = test->n; a.sn = trial->n;
 		a.tc = (const double *)test->d_c.get();
 		a.sc = (const double *)trial->d_c.get();
-		a.thr_near = (const double *)trial->d_thr.get();
+		a.thr_near = (const double *)trial->d_thr.get() + (size_t)slot * trial->n;
+		const bool skip_shared = slot != nbk::THR_NEAR && same;
+		a.t_node = skip_shared ? (const int *)test->d_tri.get() : nullptr;
+		a.s_node = skip_shared ? (const int *)trial->d_tri.get() : nullptr;
+		a.npe = trial->npe;
 		const size_t ncnt = (size_t)a.n_rows * a.n_chunks;
 		DevPtr counts, offsets, tmp;
 		int s;
@@ -628,14 +641,35 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, const nb_pol
 }
 
 // trial-sequence chunk per work-group: as long as possible (the slot
-// accumulators flush at every chunk end) while the grid keeps >= 2048
-// work-groups for the 256 CUs
+// accumulators flush at every chunk end) while the grid keeps >= 8192
+// work-groups for the 256 CUs, so that the chunks next to a tile's own, whose
+// rules are the largest, do not outlast the rest.  Single and double layer of
+// 9600 quadrilaterals with 2048 / 4096 / 8192 / 16384 work-groups 18.9 / 17.3 /
+// 16.6 / 16.5 ms, of 96 with chunks of at least 64 / 8 elements 1.65 / 0.31 ms.
 int gal_chunk(int n_tiles, int sn)
 {
 	int ch = 512;
 	const long long wg = (n_tiles + 3) / 4;
-	while (ch > 64 && wg * ((sn + ch - 1) / ch) < 2048) ch >>= 1;
+	while (ch > 8 && wg * ((sn + ch - 1) / ch) < 8192) ch >>= 1;
 	return ch;
+}
+
+// The close regular pairs that go to the wave-per-pair kernels under
+// distance-driven degrees: those inside the breakpoint from which on a table
+// gives degree 4 and more (7 points a triangle, 4 x 4 a quadrilateral).  No
+// list (null) when such pairs are many -- over 1/64 of all, beyond the 2^18
+// that a small mesh may have anyway: 64 lanes then share them better than one
+// wave each.
+int ensure_gal_near(nb_mesh *trial, nb_mesh *test, int same, int km, hipStream_t st, std::shared_ptr<NearList> *out)
+{
+	const int slot = km == nbk::SLP ? nbk::THR_1_8 : km == nbk::HSP ? nbk::THR_3_6 : nbk::THR_2_8;
+	out->reset();
+	const double total = (double)test->n * trial->n;
+	if (total >= 2147483648.0) return NB_OK;      // the list's counts are 32-bit
+	int s = ensure_near_list(trial, test, same, nb_policy{}, st, out, slot);
+	if (s) return s;
+	if ((double)(*out)->n * 64.0 > total + 16777216.0) out->reset();
+	return NB_OK;
 }
 
 // the nodal-dof layout of a mesh of triangles (GAL_CS slots per lane) or
@@ -790,6 +824,20 @@ int ensure_gq(nb_mesh *m, int N)
 	return NB_OK;
 }
 
+// the near list's kernel arguments (null list: no pairs)
+nbk::GalNear gal_near(const NearList *nl, const int *t_map, const int *s_map)
+{
+	nbk::GalNear g;
+	std::memset(&g, 0, sizeof(g));
+	if (!nl) return g;
+	g.n_pairs = nl->n;
+	g.pi = (const int *)nl->pi.get();
+	g.pj = (const int *)nl->pj.get();
+	g.t_dof = t_map;
+	g.s_dof = s_map;
+	return g;
+}
+
 // Galerkin assembly on quadrilateral meshes into a device buffer: the FP32
 // regular pass over all pairs (node-sharing pairs skipped), then on one mesh
 // the FP64 pass over the coincident, edge- and corner-adjacent pairs
@@ -848,6 +896,8 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 	const int kt = lt ? 0 : 1, ks = ls ? 0 : 1;   // layout kinds: node or element dofs
 	if (nodal && ((s = ensure_gal_layout(test, kt)) || (s = ensure_gal_layout(trial, ks)))) return s;
 	if (jb.same && (s = ensure_sing_pairs(trial))) return s;
+	std::shared_ptr<NearList> nl;
+	if (fixed_n == 0 && (s = ensure_gal_near(trial, test, jb.same, jb.km, st, &nl))) return s;
 	if (nodal && !accumulate && (s = zero())) return s;
 
 	nbk::GalQArgs a;
@@ -875,6 +925,9 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 		a.tq[N] = (const float *)test->d_gq[N].get();
 		a.sq[N] = (const float *)trial->d_gq[N].get();
 	}
+	const nbk::GalNear near = gal_near(nl.get(), t_map, s_map);
+	if (nl) a.thr_near = (const double *)trial->d_thr.get() + (size_t)(nl->mode - GAL_LIST) * trial->n;
+	const unsigned near_grid = (unsigned)((near.n_pairs + 3) / 4);
 	a.fixed_n = fixed_n;
 	a.complexity = complexity;
 	const double two_pi = 6.283185307179586476925286766559005768;
@@ -910,6 +963,31 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 			}
 		}
 #undef NB_GQ
+		NB_HIP(hipGetLastError());
+		if (near.n_pairs > 0) {
+#define NB_GQN(F, K) do { \
+		if (F == HELM && ck) { \
+			if (nodal) hipLaunchKernelGGL((galq_near_kernel<F, K, 4, (F == HELM)>), dim3(near_grid), dim3(256), 0, st, a, near); \
+			else hipLaunchKernelGGL((galq_near_kernel<F, K, 1, (F == HELM)>), dim3(near_grid), dim3(256), 0, st, a, near); \
+		} else if (nodal) hipLaunchKernelGGL((galq_near_kernel<F, K, 4>), dim3(near_grid), dim3(256), 0, st, a, near); \
+		else hipLaunchKernelGGL((galq_near_kernel<F, K, 1>), dim3(near_grid), dim3(256), 0, st, a, near); } while (0)
+			if (jb.family == NB_HELMHOLTZ) {
+				switch (jb.km) {
+				case SLP: NB_GQN(HELM, SLP); break;
+				case DLP: NB_GQN(HELM, DLP); break;
+				case DLPT: NB_GQN(HELM, DLPT); break;
+				default: NB_GQN(HELM, HSP); break;
+				}
+			} else {
+				switch (jb.km) {
+				case SLP: NB_GQN(LAP, SLP); break;
+				case DLP: NB_GQN(LAP, DLP); break;
+				case DLPT: NB_GQN(LAP, DLPT); break;
+				default: NB_GQN(LAP, HSP); break;
+				}
+			}
+#undef NB_GQN
+		}
 		NB_HIP(hipGetLastError());
 		prof_end(pe, st);
 	}
@@ -1010,6 +1088,8 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 	const int kt = lt ? 0 : 1, ks = ls ? 0 : 1;   // layout kinds: node or element dofs
 	if (nodal && ((s = ensure_gal_layout(test, kt)) || (s = ensure_gal_layout(trial, ks)))) return s;
 	if (jb.same && (s = ensure_sing_pairs(trial))) return s;
+	std::shared_ptr<NearList> nl;
+	if (jb.pol.rule != NB_RULE_FIXED && (s = ensure_gal_near(trial, test, jb.same, jb.km, st, &nl))) return s;
 	if (nodal && !accumulate && (s = zero())) return s;
 
 	const nbk::Rules *rules = nullptr;
@@ -1043,6 +1123,9 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		a.sq[d] = (const nbk::QPoint *)trial->d_qt[d].get();
 		a.qn[d] = trial->qn[d];
 	}
+	const nbk::GalNear near = gal_near(nl.get(), t_map, s_map);
+	if (nl) a.thr_near = (const double *)trial->d_thr.get() + (size_t)(nl->mode - GAL_LIST) * trial->n;
+	const unsigned near_grid = (unsigned)((near.n_pairs + 3) / 4);
 	a.fixed_degree = jb.pol.rule == NB_RULE_FIXED ? jb.pol.fixed_degree : -1;
 	const double two_pi = 6.283185307179586476925286766559005768;
 	a.k = (float)jb.k;
@@ -1083,6 +1166,31 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 			}
 		}
 #undef NB_GAL
+		NB_HIP(hipGetLastError());
+		if (near.n_pairs > 0) {
+#define NB_GALN(F, K) do { \
+		if (F == HELM && ck) { \
+			if (nodal) hipLaunchKernelGGL((galerkin_near_kernel<F, K, 3, (F == HELM)>), dim3(near_grid), dim3(256), 0, st, a, near); \
+			else hipLaunchKernelGGL((galerkin_near_kernel<F, K, 1, (F == HELM)>), dim3(near_grid), dim3(256), 0, st, a, near); \
+		} else if (nodal) hipLaunchKernelGGL((galerkin_near_kernel<F, K, 3>), dim3(near_grid), dim3(256), 0, st, a, near); \
+		else hipLaunchKernelGGL((galerkin_near_kernel<F, K, 1>), dim3(near_grid), dim3(256), 0, st, a, near); } while (0)
+			if (jb.family == NB_HELMHOLTZ) {
+				switch (jb.km) {
+				case SLP: NB_GALN(HELM, SLP); break;
+				case DLP: NB_GALN(HELM, DLP); break;
+				case DLPT: NB_GALN(HELM, DLPT); break;
+				default: NB_GALN(HELM, HSP); break;
+				}
+			} else {
+				switch (jb.km) {
+				case SLP: NB_GALN(LAP, SLP); break;
+				case DLP: NB_GALN(LAP, DLP); break;
+				case DLPT: NB_GALN(LAP, DLPT); break;
+				default: NB_GALN(LAP, HSP); break;
+				}
+			}
+#undef NB_GALN
+		}
 		NB_HIP(hipGetLastError());
 		prof_end(pe, st);
 	}

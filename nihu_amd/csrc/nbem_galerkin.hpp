@@ -53,6 +53,9 @@ struct GalArgs {
 	const double *tc, *sc;       // centres [3][n]
 	const float *tnu, *snu;      // unit normals [3][n]
 	const double *thr;           // trial distance thresholds [NTHR][sn]
+	// squared distances below which a pair's degree is left to
+	// galerkin_near_kernel, by trial element (null: every degree here)
+	const double *thr_near;
 	const QPoint *tq[NSLOT], *sq[NSLOT];
 	int qn[NSLOT];
 	const float2 *ref;           // [NSLOT][REF_MAXQ] reference points (xi, eta) of each degree's rule
@@ -118,6 +121,73 @@ __device__ __forceinline__ void atomic_add_entry64(void *out, long long idx, int
 	}
 }
 
+// One point pair's kernel value (the DLP value without its factor -r.n_y, which
+// does not depend on the trial point): trial point offset o with |o|^2, test
+// point by e = 2 (c_f - c_e - a_p) and vp = |a_p|^2 - 2 (c_f - c_e).a_p.
+template <int FAM, int KM, bool CK>
+__device__ __forceinline__ float2 gal_point(float ox, float oy, float oz, float oo, float ex, float ey, float ez, float vp,
+	float rny, const GalPair &P, float k_revf, float k, float kim)
+{
+	constexpr bool IM = FAM == HELM;
+	const float u = __builtin_fmaf(ex, ox, __builtin_fmaf(ey, oy, __builtin_fmaf(ez, oz, oo + vp)));
+	const float r2 = P.d2f + u;
+	const float rinv = __builtin_amdgcn_rsqf(r2);
+	float c = 1.0f, sn = 0.0f;
+	if (IM) {
+		const float rd = u * __builtin_amdgcn_rcpf(__builtin_fmaf(r2, rinv, P.df));   // r - d
+		const float tt = __builtin_fmaf(k_revf, rd, P.t0);
+		c = __builtin_amdgcn_cosf(tt);
+		sn = __builtin_amdgcn_sinf(tt);
+		if (CK) {
+			const float am = P.ad * __builtin_amdgcn_exp2f(kim * 1.4426950408889634f * rd);
+			c *= am;
+			sn *= am;
+		}
+	}
+	float kr, ki = 0.0f;
+	if (KM == SLP) {
+		kr = rinv * c;
+		if (IM) ki = -rinv * sn;
+	} else {
+		const float ri2 = rinv * rinv;
+		const float g3 = rinv * ri2;
+		const float Gr = g3 * c, Gi = IM ? -g3 * sn : 0.0f;
+		const float kh = k * ri2;
+		// Q = G (1 + i th): Re = Gr + k sn / r^2, Im = Gi + k c / r^2
+		float Qr = IM ? __builtin_fmaf(kh, sn, Gr) : Gr;
+		float Qi = IM ? __builtin_fmaf(kh, c, Gi) : 0.0f;
+		if (CK) {
+			const float kih = kim * ri2;
+			Qr = __builtin_fmaf(-kih, c, Qr);
+			Qi = __builtin_fmaf(kih, sn, Qi);
+		}
+		if (KM == DLP) {
+			kr = Qr; ki = Qi;
+		} else {
+			const float rnx = P.dcnx + __builtin_fmaf(ox, P.nxx, __builtin_fmaf(oy, P.nxy, oz * P.nxz));
+			if (KM == DLPT) {
+				kr = Qr * rnx; ki = Qi * rnx;
+			} else {
+				const float cf = rnx * rny * ri2;
+				// 3 Q - th^2 G with th^2 G = k^2 E = k^2 e^{-i th} / r
+				float hr, hi;
+				if (CK) {
+					const float kr2 = (k * k - kim * kim) * rinv, ki2 = 2.0f * k * kim * rinv;
+					hr = 3.0f * Qr - (kr2 * c + ki2 * sn);
+					hi = 3.0f * Qi - (ki2 * c - kr2 * sn);
+				} else {
+					const float kk = k * k * rinv;
+					hr = __builtin_fmaf(3.0f, Qr, -kk * c);
+					hi = __builtin_fmaf(3.0f, Qi, kk * sn);
+				}
+				kr = __builtin_fmaf(P.nn, Qr, -hr * cf);
+				ki = __builtin_fmaf(P.nn, Qi, -hi * cf);
+			}
+		}
+	}
+	return make_float2(kr, ki);
+}
+
 // One pair over the diadic rule: for each test point p (tp(p), per lane) the
 // sums S_b = sum_q K(x_p, y_q) w_q J_f N_b(q) / (4 pi) over the trial points
 // (wave-uniform table rows), then block[a][b] += w_p J_e N_a(p) S_b.
@@ -163,62 +233,8 @@ __device__ __forceinline__ void gal_points(TP tp, const QPoint *sq_in, const flo
 #pragma unroll UNROLL
 		for (int q = 0; q < nq; ++q) {
 			const float ox = sf[8 * q], oy = sf[8 * q + 1], oz = sf[8 * q + 2], w = sf[8 * q + 3], oo = sf[8 * q + 4];
-			const float u = __builtin_fmaf(ex, ox, __builtin_fmaf(ey, oy, __builtin_fmaf(ez, oz, oo + vp)));
-			const float r2 = P.d2f + u;
-			const float rinv = __builtin_amdgcn_rsqf(r2);
-			float c = 1.0f, sn = 0.0f;
-			if (IM) {
-				const float rd = u * __builtin_amdgcn_rcpf(__builtin_fmaf(r2, rinv, P.df));   // r - d
-				const float tt = __builtin_fmaf(k_revf, rd, P.t0);
-				c = __builtin_amdgcn_cosf(tt);
-				sn = __builtin_amdgcn_sinf(tt);
-				if (CK) {
-					const float am = P.ad * __builtin_amdgcn_exp2f(kim * 1.4426950408889634f * rd);
-					c *= am;
-					sn *= am;
-				}
-			}
-			float kr, ki = 0.0f;
-			if (KM == SLP) {
-				kr = rinv * c;
-				if (IM) ki = -rinv * sn;
-			} else {
-				const float ri2 = rinv * rinv;
-				const float g3 = rinv * ri2;
-				const float Gr = g3 * c, Gi = IM ? -g3 * sn : 0.0f;
-				const float kh = k * ri2;
-				// Q = G (1 + i th): Re = Gr + k sn / r^2, Im = Gi + k c / r^2
-				float Qr = IM ? __builtin_fmaf(kh, sn, Gr) : Gr;
-				float Qi = IM ? __builtin_fmaf(kh, c, Gi) : 0.0f;
-				if (CK) {
-					const float kih = kim * ri2;
-					Qr = __builtin_fmaf(-kih, c, Qr);
-					Qi = __builtin_fmaf(kih, sn, Qi);
-				}
-				if (KM == DLP) {
-					kr = Qr; ki = Qi;
-				} else {
-					const float rnx = P.dcnx + __builtin_fmaf(ox, P.nxx, __builtin_fmaf(oy, P.nxy, oz * P.nxz));
-					if (KM == DLPT) {
-						kr = Qr * rnx; ki = Qi * rnx;
-					} else {
-						const float cf = rnx * rny * ri2;
-						// 3 Q - th^2 G with th^2 G = k^2 E = k^2 e^{-i th} / r
-						float hr, hi;
-						if (CK) {
-							const float kr2 = (k * k - kim * kim) * rinv, ki2 = 2.0f * k * kim * rinv;
-							hr = 3.0f * Qr - (kr2 * c + ki2 * sn);
-							hi = 3.0f * Qi - (ki2 * c - kr2 * sn);
-						} else {
-							const float kk = k * k * rinv;
-							hr = __builtin_fmaf(3.0f, Qr, -kk * c);
-							hi = __builtin_fmaf(3.0f, Qi, kk * sn);
-						}
-						kr = __builtin_fmaf(P.nn, Qr, -hr * cf);
-						ki = __builtin_fmaf(P.nn, Qi, -hi * cf);
-					}
-				}
-			}
+			const float2 K = gal_point<FAM, KM, CK>(ox, oy, oz, oo, ex, ey, ez, vp, rny, P, k_revf, k, kim);
+			const float kr = K.x, ki = K.y;
 			if (NDOF == 1) {
 				S[0].x = __builtin_fmaf(kr, w, S[0].x);
 				if (IM) S[0].y = __builtin_fmaf(ki, w, S[0].y);
@@ -259,7 +275,7 @@ __device__ __forceinline__ void gal_eval_dynamic(const GalArgs &a, int e, int f,
 	const GalPair &P, float2 (&blk)[NDOF][NDOF])
 {
 	constexpr int ORDER = KM == SLP ? 1 : KM == HSP ? 3 : 2;
-	int deg = a.fixed_degree >= 0 ? a.fixed_degree : (NDOF == 3 ? 1 : 0) + table_degree<ORDER>(d2, a.thr, a.sn, f);
+	int deg = a.fixed_degree >= 0 ? a.fixed_degree : (NDOF == 3 ? 1 : 0) + table_degree<ORDER>(d2, uni(a.thr), a.sn, f);
 	deg = act ? deg : -1;
 	for (;;) {
 		const unsigned long long m = __ballot(deg >= 0);
@@ -373,7 +389,7 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 			sing = tv0 == f0 || tv0 == f1 || tv0 == f2 || tv1 == f0 || tv1 == f1 || tv1 == f2 ||
 				tv2 == f0 || tv2 == f1 || tv2 == f2;
 		}
-		const bool act = lane_ok && !sing;
+		const bool act = lane_ok && !sing && !(a.thr_near && d2 < uni(a.thr_near)[f]);
 		float2 blk[NDOF][NDOF];
 #pragma unroll
 		for (int x = 0; x < NDOF; ++x)
@@ -447,6 +463,118 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 			if (v >= 0) gal_flush(acc, lane, s, v, rnode, con, a);
 		}
 	}
+}
+
+// ---------------------------------------------------------------- close regular pairs
+
+// sum over the wave, valid in lane 63
+__device__ __forceinline__ float wave_sum63(float v)
+{
+#define NB_DPP_ADD(ctrl, rows) \
+	v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, rows, 0xf, false))
+	NB_DPP_ADD(0x111, 0xf);    // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's sum
+	NB_DPP_ADD(0x112, 0xf);
+	NB_DPP_ADD(0x114, 0xf);
+	NB_DPP_ADD(0x118, 0xf);
+	NB_DPP_ADD(0x142, 0xa);    // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+	NB_DPP_ADD(0x143, 0xc);
+#undef NB_DPP_ADD
+	return v;
+}
+
+// Pairs of a near list (test, trial element) and the dofs of their corners
+struct GalNear {
+	int n_pairs;
+	const int *pi, *pj;
+	const int *t_dof, *s_dof;    // [npe][tn], [npe][sn] (nodal)
+};
+
+// The regular pairs of the higher distance-table degrees (close, not sharing
+// a node): one wave per pair, lane = (group g, trial point q), the groups
+// sharing out the test points.  In galerkin_regular_kernel such a pair keeps
+// one lane busy with up to 19 x 19 points while its wave waits, and the chunk
+// of trial elements next to a tile's own sets the launch's time (double layer,
+// 4332 elements: 3.66 ms; 0.73 ms with these pairs taken here and chunks of 8
+// elements).  A handful of them per element, so one atomic per entry.
+template <int FAM, int KM, int NDOF, bool CK = false>
+__global__ void __launch_bounds__(256) galerkin_near_kernel(GalArgs a, GalNear l)
+{
+	const int pair = (int)__builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+	if (pair >= l.n_pairs) return;
+	const int lane = threadIdx.x & 63;
+	const int e = uni(l.pi)[pair], f = uni(l.pj)[pair];
+	constexpr int ORDER = KM == SLP ? 1 : KM == HSP ? 3 : 2;
+	const auto tc = uni(a.tc), sc = uni(a.sc);
+	const auto tnu = uni(a.tnu), snu = uni(a.snu);
+	const double dx = sc[f] - tc[e], dy = sc[a.sn + f] - tc[a.tn + e], dz = sc[2 * a.sn + f] - tc[2 * a.tn + e];
+	const double d2 = __fma_rn(dz, dz, __fma_rn(dy, dy, dx * dx));
+	const int deg = __builtin_amdgcn_readfirstlane((NDOF == 3 ? 1 : 0) + table_degree<ORDER>(d2, uni(a.thr), a.sn, f));
+	const int nq = a.qn[deg];
+	GalPair P;
+	const float dcx = (float)dx, dcy = (float)dy, dcz = (float)dz;
+	P.ex0 = 2.0f * dcx; P.ey0 = 2.0f * dcy; P.ez0 = 2.0f * dcz;
+	P.d2f = (float)d2;
+	P.df = P.t0 = 0.0f;
+	P.ad = 1.0f;
+	if (FAM == HELM) {
+		double y = __builtin_amdgcn_rsq(d2);
+		y = y * (1.5 - 0.5 * d2 * y * y);
+		const double d = d2 * y;
+		double t = d * a.k_rev;
+		t -= rint(t);
+		P.df = (float)d;
+		P.t0 = (float)t;
+		if (CK) P.ad = __builtin_amdgcn_exp2f((float)(d * (a.ki * 1.4426950408889634)));
+	}
+	P.nxx = tnu[e]; P.nxy = tnu[a.tn + e]; P.nxz = tnu[2 * a.tn + e];
+	P.nyx = snu[f]; P.nyy = snu[a.sn + f]; P.nyz = snu[2 * a.sn + f];
+	P.dcny = dcx * P.nyx + dcy * P.nyy + dcz * P.nyz;
+	P.dcnx = dcx * P.nxx + dcy * P.nxy + dcz * P.nxz;
+	P.nn = P.nxx * P.nyx + P.nxy * P.nyy + P.nxz * P.nyz;
+	const int groups = 64 / nq;
+	const int g = lane / nq, q = lane - g * nq;
+	float2 T[NDOF];
+#pragma unroll
+	for (int x = 0; x < NDOF; ++x) T[x] = zero2();
+	const float *sq = (const float *)(a.sq[deg] + (size_t)f * nq + q);
+	const float ox = sq[0], oy = sq[1], oz = sq[2], oo = sq[4];
+	const float *tq = (const float *)(a.tq[deg] + (size_t)e * nq);
+	const float2 *ref = a.ref + deg * REF_MAXQ;
+	for (int p = g < groups ? g : nq; p < nq; p += groups) {
+		const float ax = tq[8 * p], ay = tq[8 * p + 1], az = tq[8 * p + 2], aa = tq[8 * p + 4], wj = tq[8 * p + 7];
+		const float ex = __builtin_fmaf(-2.0f, ax, P.ex0);
+		const float ey = __builtin_fmaf(-2.0f, ay, P.ey0);
+		const float ez = __builtin_fmaf(-2.0f, az, P.ez0);
+		const float vp = aa - __builtin_fmaf(P.ex0, ax, __builtin_fmaf(P.ey0, ay, P.ez0 * az));
+		float rny = 0.0f;
+		if (KM & (DLP | HSP)) rny = P.dcny - __builtin_fmaf(ax, P.nyx, __builtin_fmaf(ay, P.nyy, az * P.nyz));
+		const float2 K = gal_point<FAM, KM, CK>(ox, oy, oz, oo, ex, ey, ez, vp, rny, P, a.k_revf, a.k, a.ki);
+		const float wt = KM == DLP ? -rny * wj : wj;
+		const float2 r = ref[p];
+		const float wa[3] = {NDOF == 1 ? wt : wt * (1.0f - r.x - r.y), wt * r.x, wt * r.y};
+#pragma unroll
+		for (int x = 0; x < NDOF; ++x) {
+			T[x].x = __builtin_fmaf(wa[x], K.x, T[x].x);
+			T[x].y = __builtin_fmaf(wa[x], K.y, T[x].y);
+		}
+	}
+	// the trial weights w N_b of the lane's point, then the sum over the lanes
+	// (idle lanes hold zeros)
+	const float w = sq[3], w1 = sq[5], w2 = sq[6];
+	const float wb[3] = {NDOF == 1 ? w : w - w1 - w2, w1, w2};
+#pragma unroll
+	for (int x = 0; x < NDOF; ++x)
+#pragma unroll
+		for (int y = 0; y < NDOF; ++y) {
+			const float vr = wave_sum63(T[x].x * wb[y]);
+			const float vi = FAM == HELM ? wave_sum63(T[x].y * wb[y]) : 0.0f;
+			const float re = a.alpha.x * vr - a.alpha.y * vi;
+			const float im = a.alpha.x * vi + a.alpha.y * vr;
+			if (lane != 63) continue;
+			if (NDOF == 1) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, re, im);
+			else
+				atomic_add_entry(a.out, (long long)l.s_dof[y * a.sn + f] * a.ld + l.t_dof[x * a.tn + e], a.dtype, re, im);
+		}
 }
 
 // ---------------------------------------------------------------- FP64 pass

@@ -50,6 +50,9 @@ struct GalQArgs {
 	const int *s_quad;           // trial element nodes [4][sn]
 	const double *tc, *sc;       // centres x(0, 0) [3][n]
 	const double *thr;           // trial distance thresholds [NTHR][sn]
+	// squared distances below which a pair's rule is left to galq_near_kernel,
+	// by trial element (null: every rule here)
+	const double *thr_near;
 	const float *tq[GALQ_NMAX + 1], *sq[GALQ_NMAX + 1];   // point rows by points per axis
 	int fixed_n;                 // > 0: the fixed rule's points per axis
 	int complexity;              // field complexity: 1 constant, 2 nodal
@@ -62,13 +65,100 @@ struct GalQArgs {
 	int dtype, accumulate;
 };
 
+// trial point: offset o, |o|^2, unit normal n, o.n
+struct GalqPoint { float ox, oy, oz, oo, nx, ny, nz, on; };
+
+// test point of a pair: h = c_f - c_e - a_p, vp = |a_p|^2 - 2 (c_f - c_e).a_p, unit normal, h.n
+struct GalqTest { float hx, hy, hz, vp, nx, ny, nz, rnx0; };
+
+// from the first two quarters of a point row
+template <int KM>
+__device__ __forceinline__ GalqTest galq_test(float4 t0, float4 t1, const GalPair &P)
+{
+	GalqTest x;
+	x.hx = __builtin_fmaf(0.5f, P.ex0, -t0.x);
+	x.hy = __builtin_fmaf(0.5f, P.ey0, -t0.y);
+	x.hz = __builtin_fmaf(0.5f, P.ez0, -t0.z);
+	x.vp = t0.w - __builtin_fmaf(P.ex0, t0.x, __builtin_fmaf(P.ey0, t0.y, P.ez0 * t0.z));
+	x.nx = t1.x; x.ny = t1.y; x.nz = t1.z;
+	x.rnx0 = 0.0f;
+	if (KM & (DLPT | HSP)) x.rnx0 = __builtin_fmaf(x.hx, x.nx, __builtin_fmaf(x.hy, x.ny, x.hz * x.nz));
+	return x;
+}
+
+// One point pair's kernel value without 1 / (4 pi): SLP E, DLP -Q r.n_y, DLPt
+// Q r.n_x, HSP n_x.n_y Q - (3Q - k^2 E r^2) r.n_x r.n_y / r^2 with
+// E = e^{-i th}/r, G = E/r^2, Q = G (1 + i th), th = k r, th G = k e^{-i th}/r^2.
+// CK: complex wavenumber k + i kim, the attenuation e^{kim r} on c and sn, Q
+// gains -kim r G, k^2 becomes (k + i kim)^2.
+template <int FAM, int KM, bool CK>
+__device__ __forceinline__ float2 galq_point(const GalqPoint &y, const GalqTest &x, const GalPair &P, float k_revf,
+	float k, float kim)
+{
+	constexpr bool IM = FAM == HELM;
+	const float u = __builtin_fmaf(2.0f * x.hx, y.ox, __builtin_fmaf(2.0f * x.hy, y.oy, __builtin_fmaf(2.0f * x.hz, y.oz, y.oo + x.vp)));
+	const float r2 = P.d2f + u;
+	const float rinv = __builtin_amdgcn_rsqf(r2);
+	float c = 1.0f, sn = 0.0f;
+	if (IM) {
+		const float rd = u * __builtin_amdgcn_rcpf(__builtin_fmaf(r2, rinv, P.df));   // r - d
+		const float tt = __builtin_fmaf(k_revf, rd, P.t0);
+		c = __builtin_amdgcn_cosf(tt);
+		sn = __builtin_amdgcn_sinf(tt);
+		if (CK) {
+			const float am = P.ad * __builtin_amdgcn_exp2f(kim * 1.4426950408889634f * rd);
+			c *= am;
+			sn *= am;
+		}
+	}
+	float kr, ki = 0.0f;
+	if (KM == SLP) {
+		kr = rinv * c;
+		if (IM) ki = -rinv * sn;
+	} else {
+		const float ri2 = rinv * rinv;
+		const float g3 = rinv * ri2;
+		const float Gr = g3 * c, Gi = IM ? -g3 * sn : 0.0f;
+		const float kh = k * ri2;
+		float Qr = IM ? __builtin_fmaf(kh, sn, Gr) : Gr;
+		float Qi = IM ? __builtin_fmaf(kh, c, Gi) : 0.0f;
+		if (CK) {
+			const float kih = kim * ri2;
+			Qr = __builtin_fmaf(-kih, c, Qr);
+			Qi = __builtin_fmaf(kih, sn, Qi);
+		}
+		float rny = 0.0f;
+		if (KM & (DLP | HSP)) rny = __builtin_fmaf(x.hx, y.nx, __builtin_fmaf(x.hy, y.ny, __builtin_fmaf(x.hz, y.nz, y.on)));
+		if (KM == DLP) {
+			kr = -Qr * rny; ki = -Qi * rny;
+		} else {
+			const float rnx = x.rnx0 + __builtin_fmaf(y.ox, x.nx, __builtin_fmaf(y.oy, x.ny, y.oz * x.nz));
+			if (KM == DLPT) {
+				kr = Qr * rnx; ki = Qi * rnx;
+			} else {
+				const float nn = __builtin_fmaf(x.nx, y.nx, __builtin_fmaf(x.ny, y.ny, x.nz * y.nz));
+				const float cf = rnx * rny * ri2;
+				float hr, hi;
+				if (CK) {
+					const float kr2 = (k * k - kim * kim) * rinv, ki2 = 2.0f * k * kim * rinv;
+					hr = 3.0f * Qr - (kr2 * c + ki2 * sn);
+					hi = 3.0f * Qi - (ki2 * c - kr2 * sn);
+				} else {
+					const float kk = k * k * rinv;
+					hr = __builtin_fmaf(3.0f, Qr, -kk * c);
+					hi = __builtin_fmaf(3.0f, Qi, kk * sn);
+				}
+				kr = __builtin_fmaf(nn, Qr, -hr * cf);
+				ki = __builtin_fmaf(nn, Qi, -hi * cf);
+			}
+		}
+	}
+	return make_float2(kr, ki);
+}
+
 // One pair over the diadic N x N rule: per test point p (lane's row) the
 // trial sums S_b = sum_q K(x_p, y_q) w_q J_q N_b(q) (ND = 4) or w_q J_q
-// (ND = 1), then blk[a][b] += w_p J_p N_a(p) S_b.  Kernel values without
-// 1/(4 pi): SLP E, DLP -Q r.n_y, DLPt Q r.n_x, HSP n_x.n_y Q - (3Q - k^2 E r^2)
-// r.n_x r.n_y / r^2 with E = e^{-i th}/r, G = E/r^2, Q = G (1 + i th),
-// th = k r, th G = k e^{-i th}/r^2.  CK: complex wavenumber k + i kim, the
-// attenuation e^{kim r} on c and sn, Q gains -kim r G, k^2 becomes (k + i kim)^2.
+// (ND = 1), then blk[a][b] += w_p J_p N_a(p) S_b.
 template <int FAM, int KM, int ND, bool CK = false>
 __device__ __forceinline__ void galq_points(const float *tp, const float *sq_in, int nq, const GalPair &P,
 	float k_revf, float k, float2 (&blk)[ND][ND], float kim)
@@ -80,78 +170,17 @@ __device__ __forceinline__ void galq_points(const float *tp, const float *sq_in,
 		const float4 t1 = *(const float4 *)(tp + GALQ_ROW * p + 4);
 		const float4 t2 = *(const float4 *)(tp + GALQ_ROW * p + 8);
 		const float tw = tp[GALQ_ROW * p + 12];
-		const float ax = t0.x, ay = t0.y, az = t0.z;
-		// h = c_f - c_e - a_p, ex = 2 h
-		const float hx = 0.5f * P.ex0 - ax, hy = 0.5f * P.ey0 - ay, hz = 0.5f * P.ez0 - az;
-		const float ex = 2.0f * hx, ey = 2.0f * hy, ez = 2.0f * hz;
-		const float vp = t0.w - __builtin_fmaf(P.ex0, ax, __builtin_fmaf(P.ey0, ay, P.ez0 * az));
-		const float nxx = t1.x, nxy = t1.y, nxz = t1.z;
-		float rnx0 = 0.0f;
-		if (KM & (DLPT | HSP)) rnx0 = __builtin_fmaf(hx, nxx, __builtin_fmaf(hy, nxy, hz * nxz));
+		const GalqTest x = galq_test<KM>(t0, t1, P);
 		float2 S[ND];
 #pragma unroll
 		for (int b = 0; b < ND; ++b) S[b] = zero2();
 		for (int q = 0; q < nq; ++q) {
 			const int o = GALQ_ROW * q;
 			const float ox = sf[o], oy = sf[o + 1], oz = sf[o + 2];
-			const float u = __builtin_fmaf(ex, ox, __builtin_fmaf(ey, oy, __builtin_fmaf(ez, oz, sf[o + 3] + vp)));
-			const float r2 = P.d2f + u;
-			const float rinv = __builtin_amdgcn_rsqf(r2);
-			float c = 1.0f, sn = 0.0f;
-			if (IM) {
-				const float rd = u * __builtin_amdgcn_rcpf(__builtin_fmaf(r2, rinv, P.df));   // r - d
-				const float tt = __builtin_fmaf(k_revf, rd, P.t0);
-				c = __builtin_amdgcn_cosf(tt);
-				sn = __builtin_amdgcn_sinf(tt);
-				if (CK) {
-					const float am = P.ad * __builtin_amdgcn_exp2f(kim * 1.4426950408889634f * rd);
-					c *= am;
-					sn *= am;
-				}
-			}
-			float kr, ki = 0.0f;
-			if (KM == SLP) {
-				kr = rinv * c;
-				if (IM) ki = -rinv * sn;
-			} else {
-				const float ri2 = rinv * rinv;
-				const float g3 = rinv * ri2;
-				const float Gr = g3 * c, Gi = IM ? -g3 * sn : 0.0f;
-				const float kh = k * ri2;
-				float Qr = IM ? __builtin_fmaf(kh, sn, Gr) : Gr;
-				float Qi = IM ? __builtin_fmaf(kh, c, Gi) : 0.0f;
-				if (CK) {
-					const float kih = kim * ri2;
-					Qr = __builtin_fmaf(-kih, c, Qr);
-					Qi = __builtin_fmaf(kih, sn, Qi);
-				}
-				const float nyx = sf[o + 4], nyy = sf[o + 5], nyz = sf[o + 6];
-				float rny = 0.0f;
-				if (KM & (DLP | HSP)) rny = __builtin_fmaf(hx, nyx, __builtin_fmaf(hy, nyy, __builtin_fmaf(hz, nyz, sf[o + 7])));
-				if (KM == DLP) {
-					kr = -Qr * rny; ki = -Qi * rny;
-				} else {
-					const float rnx = rnx0 + __builtin_fmaf(ox, nxx, __builtin_fmaf(oy, nxy, oz * nxz));
-					if (KM == DLPT) {
-						kr = Qr * rnx; ki = Qi * rnx;
-					} else {
-						const float nn = __builtin_fmaf(nxx, nyx, __builtin_fmaf(nxy, nyy, nxz * nyz));
-						const float cf = rnx * rny * ri2;
-						float hr, hi;
-						if (CK) {
-							const float kr2 = (k * k - kim * kim) * rinv, ki2 = 2.0f * k * kim * rinv;
-							hr = 3.0f * Qr - (kr2 * c + ki2 * sn);
-							hi = 3.0f * Qi - (ki2 * c - kr2 * sn);
-						} else {
-							const float kk = k * k * rinv;
-							hr = __builtin_fmaf(3.0f, Qr, -kk * c);
-							hi = __builtin_fmaf(3.0f, Qi, kk * sn);
-						}
-						kr = __builtin_fmaf(nn, Qr, -hr * cf);
-						ki = __builtin_fmaf(nn, Qi, -hi * cf);
-					}
-				}
-			}
+			const GalqPoint y{ox, oy, oz, sf[o + 3], KM == SLP ? 0.0f : sf[o + 4], KM == SLP ? 0.0f : sf[o + 5],
+				KM == SLP ? 0.0f : sf[o + 6], KM == SLP ? 0.0f : sf[o + 7]};
+			const float2 K = galq_point<FAM, KM, CK>(y, x, P, k_revf, k, kim);
+			const float kr = K.x, ki = K.y;
 			if (ND == 1) {
 				const float w = sf[o + 12];
 				S[0].x = __builtin_fmaf(kr, w, S[0].x);
@@ -286,7 +315,7 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 				sing = sing || tv[0] == fv || tv[1] == fv || tv[2] == fv || tv[3] == fv;
 			}
 		}
-		const bool act = lane_ok && !sing;
+		const bool act = lane_ok && !sing && !(a.thr_near && d2 < uni(a.thr_near)[f]);
 		float2 blk[ND][ND];
 #pragma unroll
 		for (int x = 0; x < ND; ++x)
@@ -309,7 +338,7 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 			}
 			// points per axis per lane; lanes are served one distinct rule at a time
 			int nsel = -1;
-			if (act) nsel = a.fixed_n > 0 ? a.fixed_n : (a.complexity + table_degree<ORDER>(d2, a.thr, a.sn, f)) / 2 + 1;
+			if (act) nsel = a.fixed_n > 0 ? a.fixed_n : (a.complexity + table_degree<ORDER>(d2, uni(a.thr), a.sn, f)) / 2 + 1;
 			for (;;) {
 				const unsigned long long m = __ballot(nsel > 0);
 				if (m == 0) break;
@@ -350,6 +379,76 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 			if (v >= 0) galq_flush(acc, lane, s, v, rnode, con, a);
 		}
 	}
+}
+
+// The regular pairs of the higher distance-table degrees (4 x 4 points an
+// element and more; close, not sharing a node): one wave per pair as in
+// galerkin_near_kernel.
+template <int FAM, int KM, int ND, bool CK = false>
+__global__ void __launch_bounds__(256) galq_near_kernel(GalQArgs a, GalNear l)
+{
+	const int pair = (int)__builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+	if (pair >= l.n_pairs) return;
+	const int lane = threadIdx.x & 63;
+	const int e = uni(l.pi)[pair], f = uni(l.pj)[pair];
+	constexpr int ORDER = KM == SLP ? 1 : KM == HSP ? 3 : 2;
+	const auto tc = uni(a.tc), sc = uni(a.sc);
+	const double dx = sc[f] - tc[e], dy = sc[a.sn + f] - tc[a.tn + e], dz = sc[2 * a.sn + f] - tc[2 * a.tn + e];
+	const double d2 = __fma_rn(dz, dz, __fma_rn(dy, dy, dx * dx));
+	const int N = __builtin_amdgcn_readfirstlane((a.complexity + table_degree<ORDER>(d2, uni(a.thr), a.sn, f)) / 2 + 1);
+	const int nq = N * N;
+	GalPair P;
+	P.ex0 = (float)(2.0 * dx); P.ey0 = (float)(2.0 * dy); P.ez0 = (float)(2.0 * dz);
+	P.d2f = (float)d2;
+	P.df = P.t0 = 0.0f;
+	P.ad = 1.0f;
+	if (FAM == HELM) {
+		double y = __builtin_amdgcn_rsq(d2);
+		y = y * (1.5 - 0.5 * d2 * y * y);
+		const double d = d2 * y;
+		double t = d * a.k_rev;
+		t -= rint(t);
+		P.df = (float)d;
+		P.t0 = (float)t;
+		if (CK) P.ad = __builtin_amdgcn_exp2f((float)(d * (a.ki * 1.4426950408889634)));
+	}
+	const int groups = 64 / nq;
+	const int g = lane / nq, q = lane - g * nq;
+	float2 T[ND];
+#pragma unroll
+	for (int x = 0; x < ND; ++x) T[x] = zero2();
+	const float4 *sr = (const float4 *)(a.sq[N] + ((size_t)f * nq + q) * GALQ_ROW);
+	const float4 s0 = sr[0], s1 = sr[1], s2 = sr[2];
+	const GalqPoint y{s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+	const float *tp = a.tq[N] + (size_t)e * nq * GALQ_ROW;
+	for (int p = g < groups ? g : nq; p < nq; p += groups) {
+		const float4 *tr = (const float4 *)(tp + GALQ_ROW * p);
+		const GalqTest x = galq_test<KM>(tr[0], tr[1], P);
+		const float4 t2 = tr[2];
+		const float2 K = galq_point<FAM, KM, CK>(y, x, P, a.k_revf, a.k, a.ki);
+		const float wa[4] = {ND == 1 ? tp[GALQ_ROW * p + 12] : t2.x, t2.y, t2.z, t2.w};
+#pragma unroll
+		for (int c = 0; c < ND; ++c) {
+			T[c].x = __builtin_fmaf(wa[c], K.x, T[c].x);
+			T[c].y = __builtin_fmaf(wa[c], K.y, T[c].y);
+		}
+	}
+	// the trial weights w J N_b of the lane's point, then the sum over the
+	// lanes (idle lanes hold zeros)
+	const float wb[4] = {ND == 1 ? ((const float *)sr)[12] : s2.x, s2.y, s2.z, s2.w};
+#pragma unroll
+	for (int c = 0; c < ND; ++c)
+#pragma unroll
+		for (int b = 0; b < ND; ++b) {
+			const float vr = wave_sum63(T[c].x * wb[b]);
+			const float vi = FAM == HELM ? wave_sum63(T[c].y * wb[b]) : 0.0f;
+			const float re = a.alpha.x * vr - a.alpha.y * vi;
+			const float im = a.alpha.x * vi + a.alpha.y * vr;
+			if (lane != 63) continue;
+			if (ND == 1) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, re, im);
+			else
+				atomic_add_entry(a.out, (long long)l.s_dof[b * a.sn + f] * a.ld + l.t_dof[c * a.tn + e], a.dtype, re, im);
+		}
 }
 
 struct GalQSingArgs {

@@ -229,8 +229,8 @@ __device__ __forceinline__ void store_entry64(void *out, long long idx, int dtyp
 
 // Regular Dunavant degree of one pair from the squared-distance thresholds of
 // the trial element: the first breakpoint x with d/R < x (nihu/tmp/interval.hpp:173-185).
-template <int ORDER>
-__device__ __forceinline__ int table_degree(double d2, const double *thr, int sn, int j)
+template <int ORDER, class THR>
+__device__ __forceinline__ int table_degree(double d2, THR thr, int sn, int j)
 {
 	if (ORDER == 1) {          // inverse<1>: 1.1 -> 6, 1.8 -> 4, 9.1 -> 2, else 0
 		if (d2 < thr[THR_1_1 * sn + j]) return 6;
@@ -1411,7 +1411,19 @@ struct ListArgs {
 	int *counts;            // [n_rows][n_chunks]
 	const int *offsets;     // exclusive scan of counts
 	int *pi, *pj;
+	// element nodes [npe][tn] / [npe][sn]: pairs that share a node are left out (null: none are)
+	const int *t_node, *s_node;
+	int npe;
 };
+
+// do test element i and trial element j have a node in common?
+__device__ __forceinline__ bool list_share_node(const ListArgs &a, int i, int j)
+{
+	for (int x = 0; x < a.npe; ++x)
+		for (int y = 0; y < a.npe; ++y)
+			if (a.t_node[x * a.tn + i] == a.s_node[y * a.sn + j]) return true;
+	return false;
+}
 
 template <bool FILL>
 __global__ void __launch_bounds__(256) near_list_kernel(ListArgs a)
@@ -1426,7 +1438,7 @@ __global__ void __launch_bounds__(256) near_list_kernel(ListArgs a)
 	int base = FILL ? a.offsets[(long long)i * a.n_chunks + ch] : 0;
 	for (int j = j0; j < j1; ++j) {
 		const double d2 = d2_pair(cix, ciy, ciz, a.sc[j], a.sc[a.sn + j], a.sc[2 * a.sn + j]);
-		if (d2 < a.thr_near[j] && !(a.same_mesh && i == j)) {
+		if (d2 < a.thr_near[j] && !(a.same_mesh && i == j) && !(a.t_node && list_share_node(a, i, j))) {
 			if (FILL) { a.pi[base + cnt] = i; a.pj[base + cnt] = j; }
 			++cnt;
 		}

@@ -73,3 +73,42 @@ def test_burton_miller_quadrilaterals(nb, orc, n_elem):
     Ar, Br = orc.assemble_bm(nodes, quads, 4.0, rows=rows)
     check(A[rows].cpu().numpy(), Ar)
     check(B[rows].cpu().numpy(), Br)
+
+
+def galerkin(nb, m, t, form, ny, k, pol=None):
+    import torch
+    out = nb.colmajor(m.dofs(form, "test"), t.dofs(form, "trial"))
+    nb.assemble(m, t, out, nb.NB_HELMHOLTZ, 0, ny, k, pol=pol, accumulate=False, formalism=form)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("form", ["galerkin_linear", "galerkin"])
+@pytest.mark.parametrize("quads", [False, True], ids=["triangles", "quadrilaterals"])
+@pytest.mark.parametrize("n_elem", [1, 2, 63, 65, 129, 701])
+def test_galerkin_nihu(nb, orc, n_elem, quads, form):
+    # test tiles, trial chunks and the wave-per-pair list with remainders
+    nodes, el = surface(n_elem, quads)
+    m = nb.Mesh(nodes, el)
+    scale = 0.0      # the single layer's at least: the double layer of one flat element is rounding
+    for ny in (0, 1):
+        ref = orc.assemble_galerkin(nodes, el, 1, 0, ny, k=3.0, linear=form == "galerkin_linear")
+        got = galerkin(nb, m, m, form, ny, 3.0)
+        scale = max(scale, np.abs(ref).max())
+        assert np.abs(got - ref).max() < 2e-6 * scale
+
+
+@pytest.mark.parametrize("quads", [False, True], ids=["triangles", "quadrilaterals"])
+def test_galerkin_mostly_close_pairs(nb, quads):
+    # a fine test mesh inside the near breakpoints of a few large trial
+    # elements: too many close pairs for a list, so the tiled pass takes every
+    # degree; a part of the mesh has few enough and takes the list.  The two
+    # evaluate the same points in other orders (points as close as these
+    # leave FP32 itself 1e-5 to 1e-4 off the oracle, whatever the pass)
+    nodes, el = surface(24300, quads)
+    coarse, cel = surface(24 if quads else 12, quads)
+    assert len(el) * len(cel) > (len(el) * len(cel) + 2 ** 24) / 64
+    t = nb.Mesh(coarse * 1.3, cel)
+    whole, part = nb.Mesh(nodes, el), nb.Mesh(nodes, np.ascontiguousarray(el[:2000]))
+    for ny in (0, 1):
+        check(galerkin(nb, part, t, "galerkin", ny, 2.0), galerkin(nb, whole, t, "galerkin", ny, 2.0)[:2000])
