@@ -373,11 +373,14 @@ struct nb_mesh {
 	// field in a pair with a nodal one)
 	struct GalLayout {
 		int tiles = 0, chunk = 0;
-		DevPtr order, elem, contrib, rows, col, fin;
+		DevPtr elem, contrib, rows, fin;
 	} glay[2];
+	// Galerkin trial sequences: in the order of glay[0], glay[1], element order
+	DevPtr d_grec[3];
 	DevPtr d_edof;                             // element dof map [npe][n]: e at every corner
 	// Galerkin singular pairs against itself (coincident pairs first)
 	int64_t sp_n = -1;
+	std::vector<double> share;                 // largest squared centre distance of an element sharing a node
 	DevPtr sp_e, sp_f, sp_info;
 	// both element types (npe = 0): the triangle part, the quadrilateral part
 	// and, per part, the element id (table row) of each of its elements
@@ -699,6 +702,65 @@ int ensure_edof(nb_mesh *m)
 	return NB_OK;
 }
 
+int ensure_sing_pairs(nb_mesh *m)
+{
+	if (m->sp_n >= 0) return NB_OK;
+	const int64_t cnt = nbg_singular_pairs_n(m->n_nodes, m->n, m->tri.data(), m->npe, nullptr, nullptr, nullptr);
+	if (cnt > 0x7fffffff) return fail(NB_ERR_RANGE, "too many singular element pairs");
+	std::vector<int32_t> pe(cnt), pf(cnt), info(cnt);
+	nbg_singular_pairs_n(m->n_nodes, m->n, m->tri.data(), m->npe, pe.data(), pf.data(), info.data());
+	int s;
+	if ((s = upload(m->sp_e, pe)) || (s = upload(m->sp_f, pf)) || (s = upload(m->sp_info, info))) return s;
+	// the farthest element (centre to centre) that shares a node with each: d2 as
+	// the kernels form it
+	m->share.assign(m->n, 0.0);
+	for (int64_t q = 0; q < cnt; ++q) {
+		double d[3];
+		for (int t = 0; t < 3; ++t) d[t] = m->c[(size_t)t * m->n + pe[q]] - m->c[(size_t)t * m->n + pf[q]];
+		const double d2 = std::fma(d[2], d[2], std::fma(d[1], d[1], d[0] * d[0]));
+		m->share[pf[q]] = std::max(m->share[pf[q]], d2);
+	}
+	m->sp_n = cnt;
+	m->bytes += cnt * 12;
+	return NB_OK;
+}
+
+// The trial sequence records of a mesh (GalRec): order, col as
+// nbg_galerkin_layout_n gives them, or null for element order without slots
+int upload_gal_rec(nb_mesh *m, int kind, const int32_t *order, const int32_t *col)
+{
+	int s;
+	if ((s = ensure_sing_pairs(m))) return s;
+	const int n = m->n, npe = m->npe;
+	const double four_pi = 4.0 * 3.141592653589793238462643383279502884;
+	// breakpoints of the distance tables of orders 1..3 (ensure_thresholds)
+	static const double near[3] = {18. / 10., 28. / 10., 36. / 10.}, far[3] = {91. / 10., 158. / 10., 223. / 10.};
+	std::vector<nbk::GalRec> rec(n);
+	for (int i = 0; i < n; ++i) {
+		nbk::GalRec &r = rec[i];
+		std::memset(&r, 0, sizeof(r));
+		const int f = order ? order[i] : i;
+		for (int t = 0; t < 3; ++t) {
+			r.c[t] = m->c[(size_t)t * n + f];
+			r.nu[t] = (float)m->nu[(size_t)t * n + f];
+			r.near[t] = nbg_threshold(m->R[f], near[t]);
+			r.far[t] = nbg_threshold(m->R[f], far[t]);
+		}
+		r.share = m->share[f];
+		// one-point weights as in the point tables (the triangles' carry 1 / (4 pi))
+		r.w1 = (float)(npe == 4 ? 4.0 * m->J[f] : 0.5 * m->J[f] / four_pi);
+		for (int c = 0; c < 4; ++c) {
+			r.node[c] = c < npe ? m->tri[(size_t)npe * f + c] : -2;
+			r.evict[c] = col && c < npe ? col[(size_t)(npe + 1) * i + c] : -1;
+		}
+		r.slots = col ? col[(size_t)(npe + 1) * i + npe] : 0;
+		r.elem = f;
+	}
+	if ((s = upload(m->d_grec[kind], rec))) return s;
+	m->bytes += (int64_t)n * sizeof(nbk::GalRec);
+	return NB_OK;
+}
+
 int ensure_gal_layout(nb_mesh *m, int kind = 0)
 {
 	nb_mesh::GalLayout &L = m->glay[kind];
@@ -718,26 +780,12 @@ int ensure_gal_layout(nb_mesh *m, int kind = 0)
 		contrib.data(), rows.data(), col.data(), fin.data()) != tiles)
 		return fail(NB_ERR_RUNTIME, "Galerkin layout");
 	int s;
-	if ((s = upload(L.order, order)) || (s = upload(L.elem, elem)) || (s = upload(L.contrib, contrib)) ||
-		(s = upload(L.rows, rows)) || (s = upload(L.col, col)) || (s = upload(L.fin, fin)))
+	if ((s = upload(L.elem, elem)) || (s = upload(L.contrib, contrib)) || (s = upload(L.rows, rows)) ||
+		(s = upload(L.fin, fin)) || (s = upload_gal_rec(m, kind, order.data(), col.data())))
 		return s;
 	L.tiles = tiles;
 	L.chunk = chunk;
-	m->bytes += (int64_t)(order.size() + elem.size() + rows.size() + contrib.size() + col.size() + fin.size()) * 4;
-	return NB_OK;
-}
-
-int ensure_sing_pairs(nb_mesh *m)
-{
-	if (m->sp_n >= 0) return NB_OK;
-	const int64_t cnt = nbg_singular_pairs_n(m->n_nodes, m->n, m->tri.data(), m->npe, nullptr, nullptr, nullptr);
-	if (cnt > 0x7fffffff) return fail(NB_ERR_RANGE, "too many singular element pairs");
-	std::vector<int32_t> pe(cnt), pf(cnt), info(cnt);
-	nbg_singular_pairs_n(m->n_nodes, m->n, m->tri.data(), m->npe, pe.data(), pf.data(), info.data());
-	int s;
-	if ((s = upload(m->sp_e, pe)) || (s = upload(m->sp_f, pf)) || (s = upload(m->sp_info, info))) return s;
-	m->sp_n = cnt;
-	m->bytes += cnt * 12;
+	m->bytes += (int64_t)(elem.size() + rows.size() + contrib.size() + fin.size()) * 4;
 	return NB_OK;
 }
 
@@ -908,16 +956,16 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 		a.t_elem = (const int *)test->glay[kt].elem.get();
 		a.t_contrib = (const uint2 *)test->glay[kt].contrib.get();
 		a.t_rows = (const int *)test->glay[kt].rows.get();
-		a.s_order = (const int *)trial->glay[ks].order.get();
-		a.s_col = (const int *)trial->glay[ks].col.get();
+		a.rec = (const nbk::GalRec *)trial->d_grec[ks].get();
 		a.s_fin = (const int *)trial->glay[ks].fin.get();
 	} else {
 		a.n_tiles = (test->n + nbk::GAL_TILE - 1) / nbk::GAL_TILE;
 		a.chunk = gal_chunk(a.n_tiles, trial->n);
+		if (!trial->d_grec[2] && (s = upload_gal_rec(trial, 2, nullptr, nullptr))) return s;
+		a.rec = (const nbk::GalRec *)trial->d_grec[2].get();
 	}
 	a.tn = test->n; a.sn = trial->n; a.same_mesh = jb.same;
 	a.t_quad = (const int *)test->d_tri.get();
-	a.s_quad = (const int *)trial->d_tri.get();
 	a.tc = (const double *)test->d_c.get();
 	a.sc = (const double *)trial->d_c.get();
 	a.thr = (const double *)trial->d_thr.get();
@@ -926,7 +974,7 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 		a.sq[N] = (const float *)trial->d_gq[N].get();
 	}
 	const nbk::GalNear near = gal_near(nl.get(), t_map, s_map);
-	if (nl) a.thr_near = (const double *)trial->d_thr.get() + (size_t)(nl->mode - GAL_LIST) * trial->n;
+	a.split = nl ? 1 : 0;
 	const unsigned near_grid = (unsigned)((near.n_pairs + 3) / 4);
 	a.fixed_n = fixed_n;
 	a.complexity = complexity;
@@ -1103,16 +1151,16 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		a.t_elem = (const int *)test->glay[kt].elem.get();
 		a.t_contrib = (const uint2 *)test->glay[kt].contrib.get();
 		a.t_rows = (const int *)test->glay[kt].rows.get();
-		a.s_order = (const int *)trial->glay[ks].order.get();
-		a.s_col = (const int *)trial->glay[ks].col.get();
+		a.rec = (const nbk::GalRec *)trial->d_grec[ks].get();
 		a.s_fin = (const int *)trial->glay[ks].fin.get();
 	} else {
 		a.n_tiles = (test->n + nbk::GAL_TILE - 1) / nbk::GAL_TILE;
 		a.chunk = gal_chunk(a.n_tiles, trial->n);
+		if (!trial->d_grec[2] && (s = upload_gal_rec(trial, 2, nullptr, nullptr))) return s;
+		a.rec = (const nbk::GalRec *)trial->d_grec[2].get();
 	}
 	a.tn = test->n; a.sn = trial->n; a.same_mesh = jb.same;
 	a.t_tri = (const int *)test->d_tri.get();
-	a.s_tri = (const int *)trial->d_tri.get();
 	a.tc = (const double *)test->d_c.get();
 	a.sc = (const double *)trial->d_c.get();
 	a.tnu = (const float *)test->d_nuf.get();
@@ -1124,7 +1172,7 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		a.qn[d] = trial->qn[d];
 	}
 	const nbk::GalNear near = gal_near(nl.get(), t_map, s_map);
-	if (nl) a.thr_near = (const double *)trial->d_thr.get() + (size_t)(nl->mode - GAL_LIST) * trial->n;
+	a.split = nl ? 1 : 0;
 	const unsigned near_grid = (unsigned)((near.n_pairs + 3) / 4);
 	a.fixed_degree = jb.pol.rule == NB_RULE_FIXED ? jb.pol.fixed_degree : -1;
 	const double two_pi = 6.283185307179586476925286766559005768;

@@ -37,6 +37,23 @@ constexpr int GAL_TILE = 64;    // test elements per wave tile
 constexpr int GAL_RMAX = 64;    // distinct nodes per wave tile (nodal fields)
 constexpr int GAL_CS = 8;       // column-node slots per lane (nodal fields)
 
+// One position of the trial sequence, read as one block through the scalar
+// cache a position ahead of its use: the element's centre, the squared
+// distances at which its pairs change treatment (share: the farthest element
+// that has a node in common with it; near, far by kernel order 1..3: below
+// near a pair has degree 4 and more above the field complexity, from far on
+// the lowest degree), unit normal, one-point weight, nodes, and for nodal dofs
+// the slot schedule (evict: the dof whose column leaves each corner's slot
+// first, -1 none; the slots packed in 5 bits each).
+struct GalRec {
+	double c[3], share, near[3], far[3];
+	float nu[3], w1;
+	int node[4], evict[4];
+	int slots, elem;
+	int pad[14];
+};
+static_assert(sizeof(GalRec) == 192, "GalRec layout");
+
 struct GalArgs {
 	int n_tiles, chunk;          // test wave tiles; trial sequence positions per chunk
 	int tn, sn;                  // element counts of test / trial mesh (SoA strides)
@@ -46,16 +63,12 @@ struct GalArgs {
 	                             //        local row, 8 bits each, 0xff: none
 	const int *t_rows;           // nodal: node of each local row (-1: unused)
 	const int *t_tri;            // test element nodes [3][tn]
-	const int *s_order;          // nodal: trial element at each sequence position
-	const int *s_col;            // nodal: [sn][4] previous slot occupant of corners 0..2, packed slots
+	const GalRec *rec;           // trial sequence [sn] (constant fields: element order)
 	const int *s_fin;            // nodal: [chunks][GAL_CS] slot occupants at the end of a chunk
-	const int *s_tri;            // trial element nodes [3][sn]
 	const double *tc, *sc;       // centres [3][n]
 	const float *tnu, *snu;      // unit normals [3][n]
 	const double *thr;           // trial distance thresholds [NTHR][sn]
-	// squared distances below which a pair's degree is left to
-	// galerkin_near_kernel, by trial element (null: every degree here)
-	const double *thr_near;
+	int split;                   // 1: the pairs below GalRec::near are left to galerkin_near_kernel
 	const QPoint *tq[NSLOT], *sq[NSLOT];
 	int qn[NSLOT];
 	const float2 *ref;           // [NSLOT][REF_MAXQ] reference points (xi, eta) of each degree's rule
@@ -294,48 +307,178 @@ __device__ __forceinline__ void gal_eval_dynamic(const GalArgs &a, int e, int f,
 	}
 }
 
-// per-lane accumulator of corner c in column slot s: acc[(s * 3 + c) * 64 + lane]
-__device__ __forceinline__ float2 *gal_acc(float2 *acc, int slot, int corner, int lane)
-{
-	return acc + (slot * 3 + corner) * GAL_TILE + lane;
-}
+// Column-slot accumulators in LDS, private to each lane: corner c of slot s at
+// acc[s * SLOT + c * 64 + lane]; the slot's last cell stays zero (the target of
+// unused contributor positions).  NPE corners per element.
+template <int NPE>
+struct GalSlots {
+	static constexpr int SLOT = NPE * GAL_TILE + 1;
 
-// add one column slot to the result and clear it: lane l sums local row l
-// over its contributors, then every lane clears its own three entries
-__device__ __forceinline__ void gal_flush(float2 *acc, int lane, int slot, int col, int rnode, uint2 con,
-	const GalArgs &a)
-{
-	float2 v = make_float2(0.0f, 0.0f);
+	// the lane's corners of a slot += v: reads, adds and writes in groups.  (LDS
+	// float atomics, which need no read, run at a small fraction of the rate of
+	// plain accesses: with them the passes took 2 to 3 times as long.)  A dof
+	// repeated within the element shares its slot, so slots follow one another.
+	template <class V>
+	static __device__ __forceinline__ void add(float2 *acc, int lane, int slot, V v)
+	{
+		float2 *p = acc + slot * SLOT + lane;
+		float2 t[NPE];
 #pragma unroll
-	for (int q = 0; q < 8; ++q) {
-		const unsigned c = ((q < 4 ? con.x : con.y) >> (8 * (q & 3))) & 255u;
-		if (c != 255u) {
-			const float2 t = *gal_acc(acc, slot, c & 3u, c >> 2);
-			v.x += t.x;
-			v.y += t.y;
+		for (int c = 0; c < NPE; ++c) t[c] = p[c * GAL_TILE];
+#pragma unroll
+		for (int c = 0; c < NPE; ++c) {
+			const float2 d = v(c);
+			p[c * GAL_TILE] = make_float2(t[c].x + d.x, t[c].y + d.y);
 		}
 	}
+
+	static __device__ __forceinline__ void clear(float2 *acc, int lane, int slot)
+	{
 #pragma unroll
-	for (int c = 0; c < 3; ++c) *gal_acc(acc, slot, c, lane) = make_float2(0.0f, 0.0f);
-	if (rnode >= 0 && (v.x != 0.0f || v.y != 0.0f)) {
-		const float re = a.alpha.x * v.x - a.alpha.y * v.y;
-		const float im = a.alpha.x * v.y + a.alpha.y * v.x;
-		atomic_add_entry(a.out, (long long)col * a.ld + rnode, a.dtype, re, im);
+		for (int c = 0; c < NPE; ++c) acc[slot * SLOT + c * GAL_TILE + lane] = make_float2(0.0f, 0.0f);
 	}
+};
+
+// The contributors of one local row, 8 bytes lane * 4 + corner (0xff: none), as
+// cell numbers of a slot in 16 bits each
+template <int NPE>
+struct GalRow {
+	unsigned cell[4];
+
+	__device__ __forceinline__ void set(uint2 con)
+	{
+#pragma unroll
+		for (int h = 0; h < 4; ++h) {
+			const unsigned two = (h < 2 ? con.x : con.y) >> (16 * (h & 1));
+			const unsigned a = two & 255u, b = (two >> 8) & 255u;
+			const unsigned ca = a == 255u ? NPE * GAL_TILE : (a & 3u) * GAL_TILE + (a >> 2);
+			const unsigned cb = b == 255u ? NPE * GAL_TILE : (b & 3u) * GAL_TILE + (b >> 2);
+			cell[h] = ca | cb << 16;
+		}
+	}
+
+	// the largest number of contributors of any row of the wave
+	__device__ __forceinline__ int used() const
+	{
+		int n = 0;
+#pragma unroll
+		for (int q = 0; q < 8; ++q)
+			if (__ballot(((cell[q >> 1] >> (16 * (q & 1))) & 0xffffu) != NPE * GAL_TILE) != 0) n = q + 1;
+		return n;
+	}
+
+	// sum of a slot's column over this row's contributors; ncon >= used()
+	__device__ __forceinline__ float2 sum(const float2 *slot, int ncon) const
+	{
+		float2 v = make_float2(0.0f, 0.0f);
+#pragma unroll
+		for (int h = 0; h < 4; ++h) {
+			if (2 * h >= ncon) break;
+			const float2 a = slot[cell[h] & 0xffffu], b = slot[cell[h] >> 16];
+			v.x += a.x;
+			v.y += a.y;
+			v.x += b.x;
+			v.y += b.y;
+		}
+		return v;
+	}
+};
+
+// Add one column slot to the result and clear it: lane l sums its local rows
+// over their contributors; the sums then change lanes through the slot's own
+// cells, so that an atomic instruction covers 32 consecutive local rows, real
+// and imaginary parts side by side (lane 2 i + c: part c of row 32 t + i, dof
+// node[t]): with the rows in the order of their dofs, neighbouring lanes hit the
+// same lines.  (The rate of the atomics bounds the launch at the low degrees:
+// 20172 triangles, single layer, one row and part per lane 14.0 ms.)
+template <int NPE, int ROWS, class ARGS>
+__device__ __forceinline__ void gal_flush(float2 *acc, int lane, int slot, int col, const GalRow<NPE> (&row)[ROWS],
+	const int (&node)[2 * ROWS], int ncon, const ARGS &a)
+{
+	float2 *sp = acc + slot * GalSlots<NPE>::SLOT;
+	float2 v[ROWS];
+#pragma unroll
+	for (int r = 0; r < ROWS; ++r) v[r] = row[r].sum(sp, ncon);
+#pragma unroll
+	for (int r = 0; r < ROWS; ++r)
+		sp[r * GAL_TILE + lane] = make_float2(a.alpha.x * v[r].x - a.alpha.y * v[r].y, a.alpha.x * v[r].y + a.alpha.y * v[r].x);
+	float part[2 * ROWS];
+#pragma unroll
+	for (int t = 0; t < 2 * ROWS; ++t) part[t] = ((const float *)sp)[t * 64 + lane];
+	GalSlots<NPE>::clear(acc, lane, slot);
+	const bool real = a.dtype == DT_F32 || a.dtype == DT_F64;
+#pragma unroll
+	for (int t = 0; t < 2 * ROWS; ++t) {
+		if (node[t] < 0 || part[t] == 0.0f || (real && (lane & 1))) continue;
+		const long long at = (long long)col * a.ld + node[t];
+		const long long idx = real ? at : 2 * at + (lane & 1);
+		if (a.dtype == DT_C64 || a.dtype == DT_F32) unsafeAtomicAdd((float *)a.out + idx, part[t]);
+		else unsafeAtomicAdd((double *)a.out + idx, (double)part[t]);
+	}
+}
+
+// One point pair whose points are the element centres (the one-point rules):
+// the kernel value from the pair's own distance, without weights or 1 / (4 pi)
+template <int FAM, int KM, bool CK>
+__device__ __forceinline__ float2 gal_centres(const GalPair &P, float rinv, float k, float kim)
+{
+	constexpr bool IM = FAM == HELM;
+	float c = 1.0f, sn = 0.0f;
+	if (IM) {
+		c = __builtin_amdgcn_cosf(P.t0);
+		sn = __builtin_amdgcn_sinf(P.t0);
+		if (CK) { c *= P.ad; sn *= P.ad; }
+	}
+	if (KM == SLP) return make_float2(rinv * c, IM ? -rinv * sn : 0.0f);
+	const float ri2 = rinv * rinv;
+	const float g3 = rinv * ri2;
+	const float Gr = g3 * c, Gi = IM ? -g3 * sn : 0.0f;
+	const float kh = k * ri2;
+	float Qr = IM ? __builtin_fmaf(kh, sn, Gr) : Gr;
+	float Qi = IM ? __builtin_fmaf(kh, c, Gi) : 0.0f;
+	if (CK) {
+		const float kih = kim * ri2;
+		Qr = __builtin_fmaf(-kih, c, Qr);
+		Qi = __builtin_fmaf(kih, sn, Qi);
+	}
+	if (KM == DLP) return make_float2(-P.dcny * Qr, -P.dcny * Qi);
+	if (KM == DLPT) return make_float2(P.dcnx * Qr, P.dcnx * Qi);
+	const float cf = P.dcnx * P.dcny * ri2;
+	float hr, hi;
+	if (CK) {
+		const float kr2 = (k * k - kim * kim) * rinv, ki2 = 2.0f * k * kim * rinv;
+		hr = 3.0f * Qr - (kr2 * c + ki2 * sn);
+		hi = 3.0f * Qi - (ki2 * c - kr2 * sn);
+	} else {
+		const float kk = k * k * rinv;
+		hr = __builtin_fmaf(3.0f, Qr, -kk * c);
+		hi = __builtin_fmaf(3.0f, Qi, kk * sn);
+	}
+	return make_float2(__builtin_fmaf(P.nn, Qr, -hr * cf), __builtin_fmaf(P.nn, Qi, -hi * cf));
 }
 
 // FIXQ > 0: fixed rule with FIXQ points per element (test points held in
 // registers); 0: any policy.  Grid: (test tiles / 4) x chunks, 256 lanes.
+//
+// With distance-driven degrees most pairs take one point each, and the kernel
+// is bound by what surrounds the evaluation: the LDS of the column slots (48 KB
+// a workgroup) leaves 3 waves per SIMD to hide the chain of loads behind a
+// trial element, so all of them sit in one record fetched a position ahead; the
+// nodes of the pair are compared only inside the record's share distance; a
+// pair of the lowest degree is one value for all nine corner pairs and needs no
+// table.
 template <int FAM, int KM, int NDOF, int FIXQ, bool CK = false>
 __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 {
-	__shared__ float2 acc_all[NDOF == 3 ? 4 * GAL_CS * 3 * GAL_TILE : 1];
+	typedef GalSlots<3> Slots;
+	__shared__ float2 acc_all[NDOF == 3 ? 4 * GAL_CS * Slots::SLOT : 1];
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	const int wg_tiles = (a.n_tiles + 3) >> 2;
 	const int tile = (int)(blockIdx.x % wg_tiles) * 4 + wave;
 	const int chunk = (int)(blockIdx.x / wg_tiles);
 	if (tile >= a.n_tiles) return;     // no block-wide barriers below
-	float2 *acc = acc_all + (NDOF == 3 ? wave * GAL_CS * 3 * GAL_TILE : 0);
+	float2 *acc = acc_all + (NDOF == 3 ? wave * GAL_CS * Slots::SLOT : 0);
+	constexpr int ORDER = KM == SLP ? 1 : KM == HSP ? 3 : 2;
 
 	int e;
 	if (NDOF == 3) e = a.t_elem[tile * GAL_TILE + lane];
@@ -346,62 +489,69 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 	GalPair P;
 	P.nxx = P.nxy = P.nxz = 0.0f;
 	if (KM & (DLPT | HSP)) { P.nxx = a.tnu[ee]; P.nxy = a.tnu[a.tn + ee]; P.nxz = a.tnu[2 * a.tn + ee]; }
-	int tv0 = -1, tv1 = -1, tv2 = -1;
-	if (a.same_mesh) { tv0 = a.t_tri[ee]; tv1 = a.t_tri[a.tn + ee]; tv2 = a.t_tri[2 * a.tn + ee]; }
-	int rnode = -1;
-	uint2 con = make_uint2(0xffffffffu, 0xffffffffu);
+	int tv[3] = {-1, -1, -1};
+	if (a.same_mesh)
+#pragma unroll
+		for (int c = 0; c < 3; ++c) tv[c] = a.t_tri[c * a.tn + ee];
+	GalRow<3> row[1];
+	int node[2] = {-1, -1};
+	int ncon = 0;
 	if (NDOF == 3) {
-		con = a.t_contrib[tile * GAL_TILE + lane];
-		rnode = a.t_rows[tile * GAL_TILE + lane];
+		row[0].set(a.t_contrib[tile * GAL_TILE + lane]);
 #pragma unroll
-		for (int s = 0; s < GAL_CS; ++s)
+		for (int t = 0; t < 2; ++t) node[t] = a.t_rows[tile * GAL_TILE + 32 * t + (lane >> 1)];
+		ncon = row[0].used();
 #pragma unroll
-			for (int c = 0; c < 3; ++c) *gal_acc(acc, s, c, lane) = make_float2(0.0f, 0.0f);
+		for (int s = 0; s < GAL_CS; ++s) Slots::clear(acc, lane, s);
+		if (lane < GAL_CS) acc[lane * Slots::SLOT + 3 * GAL_TILE] = make_float2(0.0f, 0.0f);
 	}
 	GTest tpr[FIXQ > 0 ? FIXQ : 1];
+	// weight of the test element's one-point rule, spread over the corner pairs
+	float wt1 = 0.0f;
 	if (FIXQ > 0) {
 		const float *q = (const float *)(a.tq[a.fixed_degree] + (size_t)ee * FIXQ);
 #pragma unroll
 		for (int p = 0; p < FIXQ; ++p) tpr[p] = GTest{q[8 * p], q[8 * p + 1], q[8 * p + 2], q[8 * p + 4], q[8 * p + 7]};
+	} else if (a.fixed_degree < 0) {
+		const float wj = ((const float *)(a.tq[NDOF == 3 ? 1 : 0] + ee))[7];
+		wt1 = NDOF == 3 ? wj * (1.0f / 9.0f) : wj;
 	}
 	const int i0 = chunk * a.chunk;
 	const int i1 = min(i0 + a.chunk, a.sn);
-	const auto sc = uni(a.sc);
-	const auto snu = uni(a.snu);
-	const auto stri = uni(a.s_tri);
-	const auto sord = uni(a.s_order);
-	const auto scol = uni(a.s_col);
+	const auto rec = uni(a.rec);
+	struct Head { double cx, cy, cz, share, near, far; float nx, ny, nz, w1; int v[3], ev[3], slots, f; };
+	auto head = [&](int i) {
+		const auto &r = rec[i];
+		return Head{r.c[0], r.c[1], r.c[2], r.share, r.near[ORDER - 1], r.far[ORDER - 1], r.nu[0], r.nu[1], r.nu[2], r.w1,
+			{r.node[0], r.node[1], r.node[2]}, {r.evict[0], r.evict[1], r.evict[2]}, r.slots, r.elem};
+	};
+	Head nxt = head(i0);
 	for (int i = i0; i < i1; ++i) {
-		const int f = NDOF == 3 ? sord[i] : i;
-		int sl0 = 0, sl1 = 0, sl2 = 0;
-		if (NDOF == 3) {
-			const int v0 = scol[4 * i], v1 = scol[4 * i + 1], v2 = scol[4 * i + 2], sl = scol[4 * i + 3];
-			sl0 = sl & 31; sl1 = (sl >> 5) & 31; sl2 = (sl >> 10) & 31;
-			if (v0 >= 0) gal_flush(acc, lane, sl0, v0, rnode, con, a);
-			if (v1 >= 0) gal_flush(acc, lane, sl1, v1, rnode, con, a);
-			if (v2 >= 0) gal_flush(acc, lane, sl2, v2, rnode, con, a);
+		const Head h = nxt;
+		nxt = head(i + 1 < i1 ? i + 1 : i);
+		const int f = h.f;
+		const int sl[3] = {h.slots & 31, (h.slots >> 5) & 31, (h.slots >> 10) & 31};
+		if (NDOF == 3)
+#pragma unroll
+			for (int c = 0; c < 3; ++c)
+				if (h.ev[c] >= 0) gal_flush<3, 1>(acc, lane, sl[c], h.ev[c], row, node, ncon, a);
+		const double d2 = d2_pair(cix, ciy, ciz, h.cx, h.cy, h.cz);
+		bool act = lane_ok && !(a.split && d2 < h.near);
+		if (a.same_mesh && __ballot(d2 <= h.share) != 0) {
+#pragma unroll
+			for (int c = 0; c < 3; ++c) act = act && !(tv[c] == h.v[0] || tv[c] == h.v[1] || tv[c] == h.v[2]);
 		}
-		const double cjx = sc[f], cjy = sc[a.sn + f], cjz = sc[2 * a.sn + f];
-		const double d2 = d2_pair(cix, ciy, ciz, cjx, cjy, cjz);
-		bool sing = false;
-		if (a.same_mesh) {
-			const int f0 = stri[f], f1 = stri[a.sn + f], f2 = stri[2 * a.sn + f];
-			sing = tv0 == f0 || tv0 == f1 || tv0 == f2 || tv1 == f0 || tv1 == f1 || tv1 == f2 ||
-				tv2 == f0 || tv2 == f1 || tv2 == f2;
-		}
-		const bool act = lane_ok && !sing && !(a.thr_near && d2 < uni(a.thr_near)[f]);
 		float2 blk[NDOF][NDOF];
-#pragma unroll
-		for (int x = 0; x < NDOF; ++x)
-#pragma unroll
-			for (int y = 0; y < NDOF; ++y) blk[x][y] = zero2();
+		float2 v1 = zero2();     // one-point pairs: the value of every corner pair
+		const bool low = FIXQ == 0 && a.fixed_degree < 0 && act && !(d2 < h.far);
+		const bool table = __ballot(act && !low) != 0;
 		if (__ballot(act) != 0) {
-			const float dcx = (float)(cjx - cix), dcy = (float)(cjy - ciy), dcz = (float)(cjz - ciz);
+			const float dcx = (float)(h.cx - cix), dcy = (float)(h.cy - ciy), dcz = (float)(h.cz - ciz);
 			P.ex0 = 2.0f * dcx; P.ey0 = 2.0f * dcy; P.ez0 = 2.0f * dcz;
 			P.d2f = (float)d2;
+			double y = __builtin_amdgcn_rsq(d2);
+			y = y * (1.5 - 0.5 * d2 * y * y);
 			if (FAM == HELM) {
-				double y = __builtin_amdgcn_rsq(d2);
-				y = y * (1.5 - 0.5 * d2 * y * y);
 				const double d = d2 * y;
 				double t = d * a.k_rev;
 				t -= rint(t);
@@ -414,53 +564,62 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 			P.nyx = P.nyy = P.nyz = 0.0f;
 			P.dcny = P.dcnx = P.nn = 0.0f;
 			if (KM & (DLP | HSP)) {
-				P.nyx = snu[f]; P.nyy = snu[a.sn + f]; P.nyz = snu[2 * a.sn + f];
+				P.nyx = h.nx; P.nyy = h.ny; P.nyz = h.nz;
 				P.dcny = dcx * P.nyx + dcy * P.nyy + dcz * P.nyz;
 			}
 			if (KM & (DLPT | HSP)) P.dcnx = dcx * P.nxx + dcy * P.nxy + dcz * P.nxz;
 			if (KM & HSP) P.nn = P.nxx * P.nyx + P.nxy * P.nyy + P.nxz * P.nyz;
-			if (FIXQ > 0) {
-				if (act) {
-					auto tp = [&](int p) { return tpr[p]; };
-					gal_points<FAM, KM, NDOF, FIXQ, decltype(tp), CK>(tp, a.sq[a.fixed_degree] + (size_t)f * FIXQ,
-						a.ref + a.fixed_degree * REF_MAXQ, FIXQ, P, a.k_revf, a.k, blk, a.ki);
+			if (FIXQ == 0 && low) {
+				const float2 K = gal_centres<FAM, KM, CK>(P, (float)y, a.k, a.ki);
+				const float w = wt1 * h.w1;
+				v1 = make_float2(K.x * w, K.y * w);
+			}
+			if (table) {
+#pragma unroll
+				for (int x = 0; x < NDOF; ++x)
+#pragma unroll
+					for (int z = 0; z < NDOF; ++z) blk[x][z] = zero2();
+				if (FIXQ > 0) {
+					if (act) {
+						auto tp = [&](int p) { return tpr[p]; };
+						gal_points<FAM, KM, NDOF, FIXQ, decltype(tp), CK>(tp, a.sq[a.fixed_degree] + (size_t)f * FIXQ,
+							a.ref + a.fixed_degree * REF_MAXQ, FIXQ, P, a.k_revf, a.k, blk, a.ki);
+					}
+				} else {
+					gal_eval_dynamic<FAM, KM, NDOF, CK>(a, ee, f, d2, act && !low, P, blk);
 				}
-			} else {
-				gal_eval_dynamic<FAM, KM, NDOF, CK>(a, ee, f, d2, act, P, blk);
 			}
 		}
 		if (NDOF == 1) {
-			// singular entries: zero here, the FP64 pass adds them
+			// singular entries and those of the close pairs: zero here, their passes add them
 			if (lane_ok && (act || !a.accumulate)) {
-				const float re = a.alpha.x * blk[0][0].x - a.alpha.y * blk[0][0].y;
-				const float im = a.alpha.x * blk[0][0].y + a.alpha.y * blk[0][0].x;
+				const float vr = low || !table ? v1.x : blk[0][0].x, vi = low || !table ? v1.y : blk[0][0].y;
+				const float re = a.alpha.x * vr - a.alpha.y * vi;
+				const float im = a.alpha.x * vi + a.alpha.y * vr;
 				store_entry(a.out, (long long)f * a.ld + e, a.dtype, a.accumulate, re, im);
 			}
-		} else if (act) {
+			continue;
+		}
+		if (FIXQ == 0 && low) {
+#pragma unroll
+			for (int z = 0; z < 3; ++z) Slots::add(acc, lane, sl[z], [&](int) { return v1; });
+		}
+		if (table && act && !low) {
 			// column 0 holds the sums with the trial weight w (T); N_0's is T - S_1 - S_2
 #pragma unroll
-			for (int x = 0; x < 3; ++x) {
-				blk[x][0].x -= blk[x][1].x + blk[x][2].x;
-				blk[x][0].y -= blk[x][1].y + blk[x][2].y;
+			for (int x = 0; x < NDOF; ++x) {
+				blk[x][0].x -= blk[x][NDOF > 1 ? 1 : 0].x + blk[x][NDOF > 2 ? 2 : 0].x;
+				blk[x][0].y -= blk[x][NDOF > 1 ? 1 : 0].y + blk[x][NDOF > 2 ? 2 : 0].y;
 			}
-			const int cl[3] = {sl0, sl1, sl2};
 #pragma unroll
-			for (int x = 0; x < 3; ++x)
-#pragma unroll
-				for (int y = 0; y < 3; ++y) {
-					float2 *p = gal_acc(acc, cl[y], x, lane);
-					float2 v = *p;
-					v.x += blk[x][y].x;
-					v.y += blk[x][y].y;
-					*p = v;
-				}
+			for (int z = 0; z < NDOF; ++z) Slots::add(acc, lane, sl[z], [&](int x) { return blk[NDOF > 1 ? x : 0][z]; });
 		}
 	}
 	if (NDOF == 3) {
 		const auto sfin = uni(a.s_fin);
 		for (int s = 0; s < GAL_CS; ++s) {
 			const int v = sfin[chunk * GAL_CS + s];
-			if (v >= 0) gal_flush(acc, lane, s, v, rnode, con, a);
+			if (v >= 0) gal_flush<3, 1>(acc, lane, s, v, row, node, ncon, a);
 		}
 	}
 }

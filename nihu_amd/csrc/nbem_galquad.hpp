@@ -44,15 +44,11 @@ struct GalQArgs {
 	const uint2 *t_contrib;      // nodal: [n_tiles][128] contributors lane * 4 + corner of local row r (lane r % 64)
 	const int *t_rows;           // nodal: [n_tiles][128] node of each local row (-1: unused)
 	const int *t_quad;           // test element nodes [4][tn]
-	const int *s_order;          // nodal: trial element at each sequence position
-	const int *s_col;            // nodal: [sn][5] previous slot occupant of corners 0..3, packed slots
+	const GalRec *rec;           // trial sequence [sn] (constant fields: element order)
 	const int *s_fin;            // nodal: [chunks][GALQ_CS] slot occupants at the end of a chunk
-	const int *s_quad;           // trial element nodes [4][sn]
 	const double *tc, *sc;       // centres x(0, 0) [3][n]
 	const double *thr;           // trial distance thresholds [NTHR][sn]
-	// squared distances below which a pair's rule is left to galq_near_kernel,
-	// by trial element (null: every rule here)
-	const double *thr_near;
+	int split;                   // 1: the pairs below GalRec::near are left to galq_near_kernel
 	const float *tq[GALQ_NMAX + 1], *sq[GALQ_NMAX + 1];   // point rows by points per axis
 	int fixed_n;                 // > 0: the fixed rule's points per axis
 	int complexity;              // field complexity: 1 constant, 2 nodal
@@ -90,10 +86,11 @@ __device__ __forceinline__ GalqTest galq_test(float4 t0, float4 t1, const GalPai
 // Q r.n_x, HSP n_x.n_y Q - (3Q - k^2 E r^2) r.n_x r.n_y / r^2 with
 // E = e^{-i th}/r, G = E/r^2, Q = G (1 + i th), th = k r, th G = k e^{-i th}/r^2.
 // CK: complex wavenumber k + i kim, the attenuation e^{kim r} on c and sn, Q
-// gains -kim r G, k^2 becomes (k + i kim)^2.
+// gains -kim r G, k^2 becomes (k + i kim)^2.  w: a weight that multiplies the
+// value.
 template <int FAM, int KM, bool CK>
 __device__ __forceinline__ float2 galq_point(const GalqPoint &y, const GalqTest &x, const GalPair &P, float k_revf,
-	float k, float kim)
+	float k, float kim, float w = 1.0f)
 {
 	constexpr bool IM = FAM == HELM;
 	const float u = __builtin_fmaf(2.0f * x.hx, y.ox, __builtin_fmaf(2.0f * x.hy, y.oy, __builtin_fmaf(2.0f * x.hz, y.oz, y.oo + x.vp)));
@@ -113,8 +110,9 @@ __device__ __forceinline__ float2 galq_point(const GalqPoint &y, const GalqTest 
 	}
 	float kr, ki = 0.0f;
 	if (KM == SLP) {
-		kr = rinv * c;
-		if (IM) ki = -rinv * sn;
+		const float g = rinv * w;
+		kr = g * c;
+		if (IM) ki = -g * sn;
 	} else {
 		const float ri2 = rinv * rinv;
 		const float g3 = rinv * ri2;
@@ -130,11 +128,13 @@ __device__ __forceinline__ float2 galq_point(const GalqPoint &y, const GalqTest 
 		float rny = 0.0f;
 		if (KM & (DLP | HSP)) rny = __builtin_fmaf(x.hx, y.nx, __builtin_fmaf(x.hy, y.ny, __builtin_fmaf(x.hz, y.nz, y.on)));
 		if (KM == DLP) {
-			kr = -Qr * rny; ki = -Qi * rny;
+			const float rw = rny * w;
+			kr = -Qr * rw; ki = -Qi * rw;
 		} else {
 			const float rnx = x.rnx0 + __builtin_fmaf(y.ox, x.nx, __builtin_fmaf(y.oy, x.ny, y.oz * x.nz));
 			if (KM == DLPT) {
-				kr = Qr * rnx; ki = Qi * rnx;
+				const float rw = rnx * w;
+				kr = Qr * rw; ki = Qi * rw;
 			} else {
 				const float nn = __builtin_fmaf(x.nx, y.nx, __builtin_fmaf(x.ny, y.ny, x.nz * y.nz));
 				const float cf = rnx * rny * ri2;
@@ -148,8 +148,8 @@ __device__ __forceinline__ float2 galq_point(const GalqPoint &y, const GalqTest 
 					hr = __builtin_fmaf(3.0f, Qr, -kk * c);
 					hi = __builtin_fmaf(3.0f, Qi, kk * sn);
 				}
-				kr = __builtin_fmaf(nn, Qr, -hr * cf);
-				ki = __builtin_fmaf(nn, Qi, -hi * cf);
+				kr = w * __builtin_fmaf(nn, Qr, -hr * cf);
+				ki = w * __builtin_fmaf(nn, Qi, -hi * cf);
 			}
 		}
 	}
@@ -209,54 +209,75 @@ __device__ __forceinline__ void galq_points(const float *tp, const float *sq_in,
 	}
 }
 
-// per-lane accumulator of corner c in column slot s: acc[(s * 4 + c) * 64 + lane]
-__device__ __forceinline__ float2 *galq_acc(float2 *acc, int slot, int corner, int lane)
-{
-	return acc + (slot * 4 + corner) * GAL_TILE + lane;
-}
+// The test element's points of the 2 x 2 rule in registers
+struct GalqTest2 { float ax, ay, az, aa, nx, ny, nz, w; };
 
-// add one column slot to the result and clear it: lane l sums its local rows
-// l and l + 64 over their contributors, then every lane clears its own four
-// entries
-__device__ __forceinline__ void galq_flush(float2 *acc, int lane, int slot, int col, const int (&rnode)[2],
-	const uint2 (&con)[2], const GalQArgs &a)
+// The lowest rule of nodal fields, 2 x 2 Gauss points on both elements.  The
+// shape functions at the points +-1/sqrt 3 are products of h+ = (1 + 1/sqrt 3)/2
+// and h- = (1 - 1/sqrt 3)/2 per axis, so the sums with N_b over the points are
+// two stages of h+ (v + rho v') and h+ (rho v + v'), rho = h-/h+ = 2 - sqrt 3:
+// 8 FMAs instead of 16 for the four sums of a real part; the four factors h+
+// ride on the test weights.  Replaces blk.
+template <int FAM, int KM, bool CK>
+__device__ __forceinline__ void galq_two(const GalqTest2 (&t)[4], const float *sq_in, const GalPair &P, float k_revf, float k,
+	float2 (&blk)[4][4], float kim)
 {
-	float2 v[2];
+	constexpr float RHO = 0.26794919243112270647f;
+	const auto sf = uni(sq_in);
+	// lo = v + rho u, hi = rho v + u
+	auto stage = [](float2 v, float2 u, float2 &lo, float2 &hi) {
+		lo = make_float2(__builtin_fmaf(RHO, u.x, v.x), __builtin_fmaf(RHO, u.y, v.y));
+		hi = make_float2(__builtin_fmaf(RHO, v.x, u.x), __builtin_fmaf(RHO, v.y, u.y));
+	};
+	float2 W[2][2][4];      // [test xi point][test eta node][trial corner]
 #pragma unroll
-	for (int r = 0; r < 2; ++r) {
-		v[r] = make_float2(0.0f, 0.0f);
+	for (int i = 0; i < 2; ++i) {
+		float2 U[2][4];
 #pragma unroll
-		for (int q = 0; q < 8; ++q) {
-			const unsigned c = ((q < 4 ? con[r].x : con[r].y) >> (8 * (q & 3))) & 255u;
-			if (c != 255u) {
-				const float2 t = *galq_acc(acc, slot, c & 3u, c >> 2);
-				v[r].x += t.x;
-				v[r].y += t.y;
+		for (int j = 0; j < 2; ++j) {
+			const GalqTest2 &p = t[2 * i + j];
+			const GalqTest x = galq_test<KM>(make_float4(p.ax, p.ay, p.az, p.aa), make_float4(p.nx, p.ny, p.nz, 0.0f), P);
+			float2 v[4];
+#pragma unroll
+			for (int q = 0; q < 4; ++q) {
+				const int o = GALQ_ROW * q;
+				const GalqPoint y{sf[o], sf[o + 1], sf[o + 2], sf[o + 3], KM == SLP ? 0.0f : sf[o + 4],
+					KM == SLP ? 0.0f : sf[o + 5], KM == SLP ? 0.0f : sf[o + 6], KM == SLP ? 0.0f : sf[o + 7]};
+				v[q] = galq_point<FAM, KM, CK>(y, x, P, k_revf, k, kim, sf[o + 12] * p.w);
 			}
+			// points xi outer, eta inner; corners (-,-), (+,-), (+,+), (-,+)
+			float2 m0, m1, p0, p1;
+			stage(v[0], v[1], m0, m1);
+			stage(v[2], v[3], p0, p1);
+			stage(m0, p0, U[j][0], U[j][1]);
+			stage(m1, p1, U[j][3], U[j][2]);
 		}
+#pragma unroll
+		for (int b = 0; b < 4; ++b) stage(U[0][b], U[1][b], W[i][0][b], W[i][1][b]);
 	}
 #pragma unroll
-	for (int c = 0; c < 4; ++c) *galq_acc(acc, slot, c, lane) = make_float2(0.0f, 0.0f);
-#pragma unroll
-	for (int r = 0; r < 2; ++r)
-		if (rnode[r] >= 0 && (v[r].x != 0.0f || v[r].y != 0.0f)) {
-			const float re = a.alpha.x * v[r].x - a.alpha.y * v[r].y;
-			const float im = a.alpha.x * v[r].y + a.alpha.y * v[r].x;
-			atomic_add_entry(a.out, (long long)col * a.ld + rnode[r], a.dtype, re, im);
-		}
+	for (int b = 0; b < 4; ++b) {
+		stage(W[0][0][b], W[1][0][b], blk[0][b], blk[1][b]);
+		stage(W[0][1][b], W[1][1][b], blk[3][b], blk[2][b]);
+	}
 }
 
 // Grid: (test tiles / 4) x chunks, 256 lanes (4 waves, one test tile each).
+// The lowest rule (nodal 2 x 2 points, constant one point at the centre) is
+// what most pairs take: its test points stay in registers (a lane's rows of the
+// tables are 64 different lines), its trial side comes through the scalar
+// cache; see galerkin_regular_kernel for the rest.
 template <int FAM, int KM, int ND, bool CK = false>
 __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 {
-	__shared__ float2 acc_all[ND == 4 ? 4 * GALQ_CS * 4 * GAL_TILE : 1];
+	typedef GalSlots<4> Slots;
+	__shared__ float2 acc_all[ND == 4 ? 4 * GALQ_CS * Slots::SLOT : 1];
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	const int wg_tiles = (a.n_tiles + 3) >> 2;
 	const int tile = (int)(blockIdx.x % wg_tiles) * 4 + wave;
 	const int chunk = (int)(blockIdx.x / wg_tiles);
 	if (tile >= a.n_tiles) return;     // no block-wide barriers below
-	float2 *acc = acc_all + (ND == 4 ? wave * GALQ_CS * 4 * GAL_TILE : 0);
+	float2 *acc = acc_all + (ND == 4 ? wave * GALQ_CS * Slots::SLOT : 0);
 	constexpr int ORDER = KM == SLP ? 1 : KM == HSP ? 3 : 2;
 
 	int e;
@@ -269,64 +290,77 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 	if (a.same_mesh)
 #pragma unroll
 		for (int c = 0; c < 4; ++c) tv[c] = a.t_quad[c * a.tn + ee];
-	int rnode[2] = {-1, -1};
-	uint2 con[2] = {make_uint2(0xffffffffu, 0xffffffffu), make_uint2(0xffffffffu, 0xffffffffu)};
+	GalRow<4> row[2];
+	int node[4] = {-1, -1, -1, -1};
+	int ncon = 0;
 	if (ND == 4) {
 #pragma unroll
-		for (int r = 0; r < 2; ++r) {
-			con[r] = a.t_contrib[(tile * 2 + r) * GAL_TILE + lane];
-			rnode[r] = a.t_rows[(tile * 2 + r) * GAL_TILE + lane];
-		}
+		for (int r = 0; r < 2; ++r) row[r].set(a.t_contrib[(tile * 2 + r) * GAL_TILE + lane]);
 #pragma unroll
-		for (int s = 0; s < GALQ_CS; ++s)
+		for (int t = 0; t < 4; ++t) node[t] = a.t_rows[tile * 2 * GAL_TILE + 32 * t + (lane >> 1)];
+		ncon = max(row[0].used(), row[1].used());
 #pragma unroll
-			for (int c = 0; c < 4; ++c) *galq_acc(acc, s, c, lane) = make_float2(0.0f, 0.0f);
+		for (int s = 0; s < GALQ_CS; ++s) Slots::clear(acc, lane, s);
+		if (lane < GALQ_CS) acc[lane * Slots::SLOT + 4 * GAL_TILE] = make_float2(0.0f, 0.0f);
 	}
-	const int i0 = chunk * a.chunk;
-	const int i1 = min(i0 + a.chunk, a.sn);
-	const auto sc = uni(a.sc);
-	const auto squad = uni(a.s_quad);
-	const auto sord = uni(a.s_order);
-	const auto scol = uni(a.s_col);
 	GalPair P;
 	P.nxx = P.nxy = P.nxz = 0.0f;
 	P.nyx = P.nyy = P.nyz = 0.0f;
 	P.dcny = P.dcnx = P.nn = 0.0f;
 	P.ad = 1.0f;
+	// the lowest rule's test side
+	GalqTest2 tp2[ND == 4 ? 4 : 1];
+	if (a.fixed_n <= 0) {
+		const int nq = ND == 4 ? 4 : 1;
+		const float *tp = a.tq[ND == 4 ? 2 : 1] + (size_t)ee * nq * GALQ_ROW;
+		// h+^4, h+ = (1 + 1 / sqrt 3) / 2
+		const float scale = ND == 4 ? 0.38689453417431970f : 1.0f;
+#pragma unroll
+		for (int p = 0; p < nq; ++p) {
+			const float4 t0 = *(const float4 *)(tp + GALQ_ROW * p), t1 = *(const float4 *)(tp + GALQ_ROW * p + 4);
+			tp2[p] = GalqTest2{t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, scale * tp[GALQ_ROW * p + 12]};
+		}
+		if (ND == 1) { P.nxx = tp2[0].nx; P.nxy = tp2[0].ny; P.nxz = tp2[0].nz; }
+	}
+	const int i0 = chunk * a.chunk;
+	const int i1 = min(i0 + a.chunk, a.sn);
+	const auto rec = uni(a.rec);
+	struct Head { double cx, cy, cz, share, near, far; float nx, ny, nz, w1; int v[4], ev[4], slots, f; };
+	auto head = [&](int i) {
+		const auto &r = rec[i];
+		return Head{r.c[0], r.c[1], r.c[2], r.share, r.near[ORDER - 1], r.far[ORDER - 1], r.nu[0], r.nu[1], r.nu[2], r.w1,
+			{r.node[0], r.node[1], r.node[2], r.node[3]}, {r.evict[0], r.evict[1], r.evict[2], r.evict[3]}, r.slots,
+			r.elem};
+	};
+	Head nxt = head(i0);
 	for (int i = i0; i < i1; ++i) {
-		const int f = ND == 4 ? sord[i] : i;
-		int sl[4] = {0, 0, 0, 0};
-		if (ND == 4) {
-			const int pk = scol[5 * i + 4];
+		const Head h = nxt;
+		nxt = head(i + 1 < i1 ? i + 1 : i);
+		const int f = h.f;
+		const int sl[4] = {h.slots & 31, (h.slots >> 5) & 31, (h.slots >> 10) & 31, (h.slots >> 15) & 31};
+		if (ND == 4)
 #pragma unroll
-			for (int b = 0; b < 4; ++b) {
-				sl[b] = (pk >> (5 * b)) & 31;
-				const int v = scol[5 * i + b];
-				if (v >= 0) galq_flush(acc, lane, sl[b], v, rnode, con, a);
-			}
-		}
-		const double cjx = sc[f], cjy = sc[a.sn + f], cjz = sc[2 * a.sn + f];
-		const double d2 = d2_pair(cix, ciy, ciz, cjx, cjy, cjz);
-		bool sing = false;
-		if (a.same_mesh) {
+			for (int c = 0; c < 4; ++c)
+				if (h.ev[c] >= 0) gal_flush<4, 2>(acc, lane, sl[c], h.ev[c], row, node, ncon, a);
+		const double d2 = d2_pair(cix, ciy, ciz, h.cx, h.cy, h.cz);
+		bool act = lane_ok && !(a.split && d2 < h.near);
+		if (a.same_mesh && __ballot(d2 <= h.share) != 0) {
 #pragma unroll
-			for (int c = 0; c < 4; ++c) {
-				const int fv = squad[c * a.sn + f];
-				sing = sing || tv[0] == fv || tv[1] == fv || tv[2] == fv || tv[3] == fv;
-			}
+			for (int c = 0; c < 4; ++c)
+				act = act && !(tv[c] == h.v[0] || tv[c] == h.v[1] || tv[c] == h.v[2] || tv[c] == h.v[3]);
 		}
-		const bool act = lane_ok && !sing && !(a.thr_near && d2 < uni(a.thr_near)[f]);
 		float2 blk[ND][ND];
 #pragma unroll
 		for (int x = 0; x < ND; ++x)
 #pragma unroll
 			for (int y = 0; y < ND; ++y) blk[x][y] = zero2();
 		if (__ballot(act) != 0) {
-			P.ex0 = (float)(2.0 * (cjx - cix)); P.ey0 = (float)(2.0 * (cjy - ciy)); P.ez0 = (float)(2.0 * (cjz - ciz));
+			const double dx = h.cx - cix, dy = h.cy - ciy, dz = h.cz - ciz;
+			P.ex0 = (float)(2.0 * dx); P.ey0 = (float)(2.0 * dy); P.ez0 = (float)(2.0 * dz);
 			P.d2f = (float)d2;
+			double y = __builtin_amdgcn_rsq(d2);
+			y = y * (1.5 - 0.5 * d2 * y * y);
 			if (FAM == HELM) {
-				double y = __builtin_amdgcn_rsq(d2);
-				y = y * (1.5 - 0.5 * d2 * y * y);
 				const double d = d2 * y;
 				double t = d * a.k_rev;
 				t -= rint(t);
@@ -336,24 +370,44 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 			} else {
 				P.df = 0.0f; P.t0 = 0.0f;
 			}
-			// points per axis per lane; lanes are served one distinct rule at a time
-			int nsel = -1;
-			if (act) nsel = a.fixed_n > 0 ? a.fixed_n : (a.complexity + table_degree<ORDER>(d2, uni(a.thr), a.sn, f)) / 2 + 1;
-			for (;;) {
-				const unsigned long long m = __ballot(nsel > 0);
-				if (m == 0) break;
-				const int N = __builtin_amdgcn_readlane(nsel, __ffsll((long long)m) - 1);
-				const unsigned long long msel = __ballot(nsel == N);
-				if ((msel >> __lane_id()) & 1ull) {
-					const int nq = N * N;
-					galq_points<FAM, KM, ND, CK>(a.tq[N] + (size_t)ee * nq * GALQ_ROW,
-						a.sq[N] + (size_t)f * nq * GALQ_ROW, nq, P, a.k_revf, a.k, blk, a.ki);
-					nsel = -1;
+			const bool low = a.fixed_n <= 0 && act && !(d2 < h.far);
+			if (low) {
+				if (ND == 4) {
+					galq_two<FAM, KM, CK>(reinterpret_cast<const GalqTest2 (&)[4]>(tp2), a.sq[2] + (size_t)f * 4 * GALQ_ROW, P,
+						a.k_revf, a.k, reinterpret_cast<float2 (&)[4][4]>(blk), a.ki);
+				} else {
+					// the centres of both elements, with the normals there
+					const float dcx = (float)dx, dcy = (float)dy, dcz = (float)dz;
+					P.nyx = h.nx; P.nyy = h.ny; P.nyz = h.nz;
+					if (KM & (DLP | HSP)) P.dcny = dcx * h.nx + dcy * h.ny + dcz * h.nz;
+					if (KM & (DLPT | HSP)) P.dcnx = dcx * P.nxx + dcy * P.nxy + dcz * P.nxz;
+					if (KM & HSP) P.nn = P.nxx * h.nx + P.nxy * h.ny + P.nxz * h.nz;
+					const float2 K = gal_centres<FAM, KM, CK>(P, (float)y, a.k, a.ki);
+					const float w = tp2[0].w * h.w1;
+					blk[0][0] = make_float2(K.x * w, K.y * w);
+				}
+			}
+			if (__ballot(act && !low) != 0) {
+				// points per axis per lane; lanes are served one distinct rule at a time
+				int nsel = -1;
+				if (act && !low)
+					nsel = a.fixed_n > 0 ? a.fixed_n : (a.complexity + table_degree<ORDER>(d2, uni(a.thr), a.sn, f)) / 2 + 1;
+				for (;;) {
+					const unsigned long long m = __ballot(nsel > 0);
+					if (m == 0) break;
+					const int N = __builtin_amdgcn_readlane(nsel, __ffsll((long long)m) - 1);
+					const unsigned long long msel = __ballot(nsel == N);
+					if ((msel >> __lane_id()) & 1ull) {
+						const int nq = N * N;
+						galq_points<FAM, KM, ND, CK>(a.tq[N] + (size_t)ee * nq * GALQ_ROW,
+							a.sq[N] + (size_t)f * nq * GALQ_ROW, nq, P, a.k_revf, a.k, blk, a.ki);
+						nsel = -1;
+					}
 				}
 			}
 		}
 		if (ND == 1) {
-			// singular entries: zero here, the FP64 pass adds them
+			// singular entries and those of the close pairs: zero here, their passes add them
 			if (lane_ok && (act || !a.accumulate)) {
 				const float re = a.alpha.x * blk[0][0].x - a.alpha.y * blk[0][0].y;
 				const float im = a.alpha.x * blk[0][0].y + a.alpha.y * blk[0][0].x;
@@ -361,22 +415,14 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 			}
 		} else if (act) {
 #pragma unroll
-			for (int x = 0; x < ND; ++x)
-#pragma unroll
-				for (int y = 0; y < ND; ++y) {
-					float2 *p = galq_acc(acc, sl[y], x, lane);
-					float2 v = *p;
-					v.x += blk[x][y].x;
-					v.y += blk[x][y].y;
-					*p = v;
-				}
+			for (int y = 0; y < ND; ++y) Slots::add(acc, lane, sl[y], [&](int x) { return blk[ND > 1 ? x : 0][y]; });
 		}
 	}
 	if (ND == 4) {
 		const auto sfin = uni(a.s_fin);
 		for (int s = 0; s < GALQ_CS; ++s) {
 			const int v = sfin[chunk * GALQ_CS + s];
-			if (v >= 0) galq_flush(acc, lane, s, v, rnode, con, a);
+			if (v >= 0) gal_flush<4, 2>(acc, lane, s, v, row, node, ncon, a);
 		}
 	}
 }

@@ -51,7 +51,7 @@ Tiles make_tiles(const std::vector<int> &order, const int32_t *tri, int npe, int
 	Tiles t;
 	const int n = (int)order.size();
 	int pos = 0;
-	std::vector<int> rows;
+	std::vector<int> rows, by_dof;
 	std::vector<std::vector<int> > con;
 	while (pos < n) {
 		rows.clear();
@@ -96,13 +96,18 @@ Tiles make_tiles(const std::vector<int> &order, const int32_t *tri, int npe, int
 			++cnt;
 		}
 		for (int l = 0; l < TILE; ++l) t.elem.push_back(l < cnt ? order[pos + l] : -1);
+		// local rows by ascending dof: a flushed column then touches few lines of
+		// the result (5 to 13 runs of consecutive dofs a tile instead of 40 to 80)
+		by_dof.resize(rows.size());
+		for (int l = 0; l < (int)rows.size(); ++l) by_dof[l] = l;
+		std::sort(by_dof.begin(), by_dof.end(), [&](int a, int b) { return rows[a] < rows[b]; });
 		for (int l = 0; l < rpl * TILE; ++l) {
-			t.rows.push_back(l < (int)rows.size() ? rows[l] : -1);
+			t.rows.push_back(l < (int)rows.size() ? rows[by_dof[l]] : -1);
 			uint32_t w[2] = {0xffffffffu, 0xffffffffu};
 			if (l < (int)rows.size())
-				for (int q = 0; q < (int)con[l].size(); ++q) {
+				for (int q = 0; q < (int)con[by_dof[l]].size(); ++q) {
 					w[q >> 2] &= ~(0xffu << (8 * (q & 3)));
-					w[q >> 2] |= (uint32_t)con[l][q] << (8 * (q & 3));
+					w[q >> 2] |= (uint32_t)con[by_dof[l]][q] << (8 * (q & 3));
 				}
 			t.contrib.push_back(w[0]);
 			t.contrib.push_back(w[1]);
