@@ -843,6 +843,16 @@ struct Job {
 	int passes = 3;
 };
 
+// Burton-Miller entries evaluated directly (bm_regular_kernel, triangles):
+// distance-driven degrees, a real wavenumber and an imaginary alpha, as -i/k is;
+// any other alpha needs the kernels' separate sums.  20480 triangles 1.65 -> 1.51
+// ms, 8748 0.48 -> 0.47, 20172 (columns off the line grid) 1.87 -> 1.89; on
+// quadrilaterals it gave nothing (20184: 1.64 -> 1.61, 4374: 0.175 -> 0.187 ms).
+bool bm_direct(const Job &jb)
+{
+	return jb.mode == nbk::OUT_BM && jb.pol.rule == NB_RULE_NIHU && jb.ki == 0.0 && jb.alpha.re == 0.0;
+}
+
 // element nodes [npe][n] on the device (quadrilateral meshes upload them
 // on first use)
 int ensure_elem_nodes(nb_mesh *m)
@@ -1857,7 +1867,10 @@ int run_device(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int
 		else if (mapped) hipLaunchKernelGGL((regular_kernel<F, K, M, Q, true>), dim3(grid), dim3(256), 0, st, a); \
 		else hipLaunchKernelGGL((regular_kernel<F, K, M, Q, false>), dim3(grid), dim3(256), 0, st, a); } while (0)
 		if (jb.mode == OUT_BM) {
-			if (fix7) NB_RG(HELM, ALL4, OUT_BM, 7);
+			if (bm_direct(jb)) {
+				if (mapped) hipLaunchKernelGGL((bm_regular_kernel<true>), dim3(grid), dim3(256), 0, st, a);
+				else hipLaunchKernelGGL((bm_regular_kernel<false>), dim3(grid), dim3(256), 0, st, a);
+			} else if (fix7) NB_RG(HELM, ALL4, OUT_BM, 7);
 			else NB_RG(HELM, ALL4, OUT_BM, 0);
 		} else if (jb.family == NB_HELMHOLTZ) {
 			switch (jb.km) {

@@ -596,7 +596,7 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 				const float vr = low || !table ? v1.x : blk[0][0].x, vi = low || !table ? v1.y : blk[0][0].y;
 				const float re = a.alpha.x * vr - a.alpha.y * vi;
 				const float im = a.alpha.x * vi + a.alpha.y * vr;
-				store_entry(a.out, (long long)f * a.ld + e, a.dtype, a.accumulate, re, im);
+				store_row(a.out, (long long)f * a.ld, e, a.dtype, a.accumulate, re, im);
 			}
 			continue;
 		}

@@ -411,7 +411,7 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 			if (lane_ok && (act || !a.accumulate)) {
 				const float re = a.alpha.x * blk[0][0].x - a.alpha.y * blk[0][0].y;
 				const float im = a.alpha.x * blk[0][0].y + a.alpha.y * blk[0][0].x;
-				store_entry(a.out, (long long)f * a.ld + e, a.dtype, a.accumulate, re, im);
+				store_row(a.out, (long long)f * a.ld, e, a.dtype, a.accumulate, re, im);
 			}
 		} else if (act) {
 #pragma unroll

@@ -212,8 +212,8 @@ __device__ __forceinline__ void gauss_groups(const GaussArgs &a, int j, int nS, 
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(256) gauss_regular_kernel(GaussArgs a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int r = tile_r * 256 + threadIdx.x;
 	const bool row_ok = r < a.n_rows;
 	const int rr = row_ok ? r : a.n_rows - 1;
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(256) gauss_regular_kernel(GaussArgs a)
 					const int kk = (KM & SLP) ? 0 : (KM & DLP) ? 1 : (KM & DLPT) ? 2 : 3;
 					const float re = a.alpha.x * K[dd][kk].x - a.alpha.y * K[dd][kk].y;
 					const float im = a.alpha.x * K[dd][kk].y + a.alpha.y * K[dd][kk].x;
-					store_entry(a.out0, col + r, a.dtype, a.accumulate, re, im);
+					store_row(a.out0, col, r, a.dtype, a.accumulate, re, im);
 				} else {
 					const float ar = a.alpha.x * K[dd][3].x - a.alpha.y * K[dd][3].y + K[dd][1].x;
 					const float ai = a.alpha.x * K[dd][3].y + a.alpha.y * K[dd][3].x + K[dd][1].y;
@@ -606,8 +606,8 @@ __device__ __forceinline__ void gauss_eval64(const Gauss64Args &a, int j, int n,
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(256) gauss_regular64_kernel(Gauss64Args a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int r = tile_r * 256 + threadIdx.x;
 	if (r >= a.n_rows) return;
 	const int ie = a.nodes == GDOF ? r >> 2 : r;

@@ -122,6 +122,42 @@ __device__ __forceinline__ T *entry_ptr(void *out, long long col, unsigned row_b
 	return (T *)((char *)out + col * (long long)sizeof(T) + row_bytes);
 }
 
+// Result stores of a wave whose lanes hold 64 consecutive rows of a column go
+// out non-temporally: the matrix does not fit the caches, and plain stores held
+// the waves up in the L2.  Burton-Miller with distance-driven degrees, regular
+// pass: 20480 triangles 2.02 -> 1.56 ms (1.32 without any store), 20184
+// quadrilaterals, whose columns do not start on a line, 2.1 -> 1.6 ms (plain
+// stores for the lines that two waves share: 2.0 ms).
+__device__ __forceinline__ void stream_store(float *p, float v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ void stream_store(double *p, double v) { __builtin_nontemporal_store(v, p); }
+
+__device__ __forceinline__ void stream_store(float2 *p, float2 v)
+{
+	typedef float V __attribute__((ext_vector_type(2)));
+	__builtin_nontemporal_store(V{v.x, v.y}, (V *)p);
+}
+
+__device__ __forceinline__ void stream_store(double2 *p, double2 v)
+{
+	typedef double V __attribute__((ext_vector_type(2)));
+	__builtin_nontemporal_store(V{v.x, v.y}, (V *)p);
+}
+
+// The (row tile, column tile) of a workgroup.  Workgroups go round the 8 XCDs by
+// their number; in a large grid each XCD takes a contiguous range of the tiles,
+// rows first, so that the tiles whose stores share lines run on one XCD, one
+// after the other (columns off the line grid, 20172 triangles, 199000
+// workgroups: 2.02 -> 1.88 ms with the non-temporal stores; 1944
+// quadrilaterals, 15500 workgroups: 62 -> 84 us, so small grids keep their
+// order).
+__device__ __forceinline__ void tile_of_block(int row_tiles, int &tile_r, int &tile_c)
+{
+	const unsigned n = gridDim.x, xcd = blockIdx.x & 7u;
+	const unsigned t = n < 32768u ? blockIdx.x : xcd * (n >> 3) + min(xcd, n & 7u) + (blockIdx.x >> 3);
+	tile_r = (int)(t % (unsigned)row_tiles);
+	tile_c = (int)(t / (unsigned)row_tiles);
+}
+
 __device__ __forceinline__ void store_entry(void *out, long long idx, int dtype, int accumulate, float re, float im)
 {
 	switch (dtype) {
@@ -155,47 +191,50 @@ __device__ __forceinline__ void store_entry(void *out, long long idx, int dtype,
 // compiler would otherwise sink the B sums past the A store and keep the
 // per-point terms alive, costing registers and occupancy).  With accumulate
 // the A entry is written before the B entry is read, as two single stores would.
+template <class T>
+__device__ __forceinline__ void store_two(void *out0, void *out1, long long col, unsigned row_bytes, int accumulate, T u, T v)
+{
+	T *p = entry_ptr<T>(out0, col, row_bytes), *q = entry_ptr<T>(out1, col, row_bytes);
+	if (accumulate) {
+		const T a = *p;
+		*p = a + u;
+		const T b = *q;
+		*q = b + v;
+	} else {
+		stream_store(p, u);
+		stream_store(q, v);
+	}
+}
+
 __device__ __forceinline__ void store_pair(void *out0, void *out1, long long col, int row, int dtype, int accumulate,
 	float ar, float ai, float br, float bi)
 {
 	const unsigned rb = (unsigned)row * dtype_size(dtype);
 	switch (dtype) {
-	case DT_C64: {
-		float2 *p = entry_ptr<float2>(out0, col, rb), *q = entry_ptr<float2>(out1, col, rb);
-		if (accumulate) {
-			const float2 u = *p;
-			*p = make_float2(u.x + ar, u.y + ai);
-			const float2 v = *q;
-			*q = make_float2(v.x + br, v.y + bi);
-		} else {
-			*p = make_float2(ar, ai);
-			*q = make_float2(br, bi);
-		}
-		break;
+	case DT_C64: store_two(out0, out1, col, rb, accumulate, make_float2(ar, ai), make_float2(br, bi)); break;
+	case DT_C128: store_two(out0, out1, col, rb, accumulate, make_double2(ar, ai), make_double2(br, bi)); break;
+	case DT_F32: store_two(out0, out1, col, rb, accumulate, ar, br); break;
+	default: store_two(out0, out1, col, rb, accumulate, (double)ar, (double)br); break;
 	}
-	case DT_C128: {
-		double2 *p = entry_ptr<double2>(out0, col, rb), *q = entry_ptr<double2>(out1, col, rb);
-		if (accumulate) {
-			const double2 u = *p;
-			*p = make_double2(u.x + ar, u.y + ai);
-			const double2 v = *q;
-			*q = make_double2(v.x + br, v.y + bi);
-		} else {
-			*p = make_double2(ar, ai);
-			*q = make_double2(br, bi);
-		}
-		break;
-	}
-	case DT_F32: {
-		float *p = entry_ptr<float>(out0, col, rb), *q = entry_ptr<float>(out1, col, rb);
-		if (accumulate) { *p += ar; *q += br; } else { *p = ar; *q = br; }
-		break;
-	}
-	default: {
-		double *p = entry_ptr<double>(out0, col, rb), *q = entry_ptr<double>(out1, col, rb);
-		if (accumulate) { *p += ar; *q += br; } else { *p = ar; *q = br; }
-		break;
-	}
+}
+
+// one entry of a wave's 64 consecutive rows (store_entry otherwise)
+template <class T>
+__device__ __forceinline__ void store_one(void *out, long long col, unsigned row_bytes, int accumulate, T v)
+{
+	T *p = entry_ptr<T>(out, col, row_bytes);
+	if (accumulate) *p = *p + v;
+	else stream_store(p, v);
+}
+
+__device__ __forceinline__ void store_row(void *out, long long col, int row, int dtype, int accumulate, float re, float im)
+{
+	const unsigned rb = (unsigned)row * dtype_size(dtype);
+	switch (dtype) {
+	case DT_C64: store_one(out, col, rb, accumulate, make_float2(re, im)); break;
+	case DT_C128: store_one(out, col, rb, accumulate, make_double2(re, im)); break;
+	case DT_F32: store_one(out, col, rb, accumulate, re); break;
+	default: store_one(out, col, rb, accumulate, (double)re); break;
 	}
 }
 
@@ -503,8 +542,8 @@ __device__ __forceinline__ int table_degree_rec(double d2, const double (&t)[NTH
 template <int FAM, int KM, int MODE, int FIXQ, bool MAP, bool CK = false>
 __global__ void __launch_bounds__(256) regular_kernel(RegArgs a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int i = tile_r * 256 + threadIdx.x;
 	const bool row_ok = i < a.n_rows;
 	const int ii = row_ok ? i : a.n_rows - 1;
@@ -601,7 +640,7 @@ __global__ void __launch_bounds__(256) regular_kernel(RegArgs a)
 				const int kk = (KM & SLP) ? 0 : (KM & DLP) ? 1 : (KM & DLPT) ? 2 : 3;
 				const float re = a.alpha.x * K[kk].x - a.alpha.y * K[kk].y;
 				const float im = a.alpha.x * K[kk].y + a.alpha.y * K[kk].x;
-				store_entry(a.out0, col + orow, a.dtype, a.accumulate, re, im);
+				store_row(a.out0, col, orow, a.dtype, a.accumulate, re, im);
 			} else {
 				// A = alpha D + H, B = G + alpha Ht
 				const float ar = a.alpha.x * K[3].x - a.alpha.y * K[3].y + K[1].x;
@@ -610,6 +649,208 @@ __global__ void __launch_bounds__(256) regular_kernel(RegArgs a)
 				const float bi = K[0].y + a.alpha.x * K[2].y + a.alpha.y * K[2].x;
 				store_pair(a.out0, a.out1, col, orow, a.dtype, a.accumulate, ar, ai, br, bi);
 			}
+		}
+	}
+}
+
+// ---------------------------------------------------------------- Burton-Miller with alpha = i ai
+
+// The Burton-Miller pair of entries evaluated directly, for an imaginary alpha
+// (-i/k, the composition's own): per point, with a = r.n_y, b = r.n_x,
+// nn = n_x.n_y, th = k r, G = w / r^3, b' = ai b, nn' = ai nn and
+// beta' = nn' - 3 a b' / r^2,
+//   A / (G e^{-i th}) = [-beta' th - a] + i [beta' + a k^2 b' - a th]
+//   B / (G e^{-i th}) = [r^2 - b' th] + i b'
+// (A = alpha D + H, B = G + alpha Ht with the kernels of add_point).  Two real
+// coefficients per entry replace the six complex sums and their combination.
+// Distance-driven degrees give each kernel group (SLP r^2; the double layers a
+// and b'; HSP beta' and a k^2 b') its own rule; S, D, H are 1 or 0 as the point
+// serves the group.
+struct BmPair {
+	float dcx, dcy, dcz;         // c_j - c_i
+	float d2f, df, t0, rinv;     // |c_j - c_i|^2, |c_j - c_i|, reduced phase, 1 / |c_j - c_i|
+	float av, nn, b0;            // at the centre of the trial element: a, n_x.n_y, b
+	float k, k2, ai;
+};
+
+struct BmEntry { float ar, ai, br, bi; };
+
+// wave-wide "any" without materialising the predicate as an integer
+__device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
+
+__device__ __forceinline__ void bm_add(float c, float sn, float th, float w, float rinv, float X, float Y, float U, float V,
+	BmEntry &e)
+{
+	const float g = (w * rinv) * (rinv * rinv);
+	const float gc = g * c, gs = g * sn;
+	e.ar = __builtin_fmaf(X, gc, __builtin_fmaf(Y, gs, e.ar));
+	e.ai = __builtin_fmaf(Y, gc, __builtin_fmaf(-X, gs, e.ai));
+	e.br = __builtin_fmaf(U, gc, __builtin_fmaf(V, gs, e.br));
+	e.bi = __builtin_fmaf(V, gc, __builtin_fmaf(-U, gs, e.bi));
+}
+
+// the centre of the trial element, every group (one-point rules)
+__device__ __forceinline__ void bm_far(const BmPair &p, float w1, BmEntry &e)
+{
+	const float c = __builtin_amdgcn_cosf(p.t0), sn = __builtin_amdgcn_sinf(p.t0);
+	const float th = p.k * p.df, bp = p.ai * p.b0;
+	const float beta = __builtin_fmaf(-3.0f * p.av, bp * (p.rinv * p.rinv), p.ai * p.nn);
+	bm_add(c, sn, th, w1, p.rinv, __builtin_fmaf(-beta, th, -p.av),
+		__builtin_fmaf(p.av, __builtin_fmaf(p.k2, bp, -th), beta), __builtin_fmaf(-bp, th, p.d2f), bp, e);
+}
+
+// the centre for the groups of S, D, H
+__device__ __forceinline__ void bm_far_masked(const BmPair &p, float w1, float S, float D, float H, BmEntry &e)
+{
+	const float c = __builtin_amdgcn_cosf(p.t0), sn = __builtin_amdgcn_sinf(p.t0);
+	const float th = p.k * p.df, bp = p.ai * p.b0;
+	const float beta = H * __builtin_fmaf(-3.0f * p.av, bp * (p.rinv * p.rinv), p.ai * p.nn);
+	const float aD = D * p.av, bD = D * bp, aH = H * p.av;
+	bm_add(c, sn, th, w1, p.rinv, __builtin_fmaf(-beta, th, -aD),
+		__builtin_fmaf(aH, p.k2 * bp, __builtin_fmaf(-aD, th, beta)), __builtin_fmaf(-bD, th, S * p.d2f), bD, e);
+}
+
+// a point off the centre, the hypersingular group and those of S, D: offset o
+// with |o|^2, weight w, a and n_x.n_y there
+__device__ __forceinline__ void bm_point(const BmPair &p, float u, float w, float a, float b, float nn, float k_revf, float S,
+	float D, BmEntry &e)
+{
+	const float r2 = p.d2f + u;
+	const float rinv = __builtin_amdgcn_rsqf(r2);
+	const float r = r2 * rinv;
+	const float t = __builtin_fmaf(k_revf, u * __builtin_amdgcn_rcpf(r + p.df), p.t0);
+	const float c = __builtin_amdgcn_cosf(t), sn = __builtin_amdgcn_sinf(t);
+	const float th = p.k * r, bp = p.ai * b;
+	const float beta = __builtin_fmaf(-3.0f * a, bp * (rinv * rinv), p.ai * nn);
+	const float aD = D * a, bD = D * bp;
+	bm_add(c, sn, th, w, rinv, __builtin_fmaf(-beta, th, -aD), __builtin_fmaf(a, p.k2 * bp, __builtin_fmaf(-aD, th, beta)),
+		__builtin_fmaf(-bD, th, S * r2), bD, e);
+}
+
+// A wave whose pairs all lie beyond 3.6 R takes the centre and the 3-point rule
+// only: degree 2 for SLP inside 9.1 R, the double layers inside 15.8 R and HSP
+// inside 22.3 R.  inS, inD, inH: this lane is inside those.
+__device__ __forceinline__ void bm_mid(const BmPair &p, float nxx, float nxy, float nxz, const QPoint *q3, float w1, float k_revf,
+	bool inS, bool inD, bool inH, BmEntry &e)
+{
+	const float S = inS ? 1.0f : 0.0f, D = inD ? 1.0f : 0.0f, H = inH ? 1.0f : 0.0f;
+	bm_far_masked(p, w1, 1.0f - S, 1.0f - D, 1.0f - H, e);
+	if (!inH) return;
+	const auto qf = uni((const float *)q3);
+	const float dcx2 = 2.0f * p.dcx, dcy2 = 2.0f * p.dcy, dcz2 = 2.0f * p.dcz;
+#pragma unroll
+	for (int q = 0; q < 3; ++q) {
+		const float ox = qf[8 * q], oy = qf[8 * q + 1], oz = qf[8 * q + 2], w = qf[8 * q + 3], oo = qf[8 * q + 4];
+		const float u = __builtin_fmaf(dcx2, ox, __builtin_fmaf(dcy2, oy, __builtin_fmaf(dcz2, oz, oo)));
+		const float b = __builtin_fmaf(oz, nxz, __builtin_fmaf(oy, nxy, __builtin_fmaf(ox, nxx, p.b0)));
+		// the trial element is flat: a and n_x.n_y are the centre's
+		bm_point(p, u, w, p.av, b, p.nn, k_revf, S, D, e);
+	}
+}
+
+// Close pairs: every degree of the tables, one at a time (eval_groups)
+__device__ __forceinline__ void bm_close(const RegArgs &a, int j, bool act, double d2, const double (&t)[NTHR], const BmPair &b,
+	float nxx, float nxy, float nxz, float w1, float k_revf, BmEntry &e)
+{
+	PairCtx p;
+	p.dcx = b.dcx; p.dcy = b.dcy; p.dcz = b.dcz;
+	p.d2f = b.d2f; p.df = b.df; p.t0 = b.t0;
+	p.nxx = nxx; p.nxy = nxy; p.nxz = nxz;
+	p.b0 = b.b0;
+	const int fc = a.field_complexity;
+	float2 s[6] = {zero2(), zero2(), zero2(), zero2(), zero2(), zero2()};
+	eval_groups<HELM, ALL4>(a, j, act ? fc + table_degree_rec<1>(d2, t) : -1, act ? fc + table_degree_rec<2>(d2, t) : -1,
+		act ? fc + table_degree_rec<3>(d2, t) : -1, p, w1, b.rinv, b.k, k_revf, s);
+	float2 K[4];
+	kernel_values<HELM, ALL4>(s, b.av, b.nn, b.k, true, K);
+	e.ar = K[1].x - b.ai * K[3].y;
+	e.ai = K[1].y + b.ai * K[3].x;
+	e.br = K[0].x - b.ai * K[2].y;
+	e.bi = K[0].y + b.ai * K[2].x;
+}
+
+// The geometry of a pair that does not depend on the wavenumber
+__device__ __forceinline__ void bm_geometry(double dxd, double dyd, double dzd, double d2, float nxx, float nxy, float nxz,
+	float nyx, float nyy, float nyz, BmPair &p, double &d)
+{
+	p.dcx = (float)dxd; p.dcy = (float)dyd; p.dcz = (float)dzd;
+	p.d2f = (float)d2;
+	// d and 1/d in FP64 from the hardware reciprocal square root and one Newton step
+	double y = __builtin_amdgcn_rsq(d2);
+	y = y * (1.5 - 0.5 * d2 * y * y);
+	d = d2 * y;
+	p.rinv = (float)y;
+	p.df = (float)d;
+	p.av = p.dcx * nyx + p.dcy * nyy + p.dcz * nyz;
+	p.nn = nxx * nyx + nxy * nyy + nxz * nyz;
+	p.b0 = p.dcx * nxx + p.dcy * nxy + p.dcz * nxz;
+}
+
+__device__ __forceinline__ void bm_wave(BmPair &p, double d, double k_rev, float k, float ai)
+{
+	double tt = d * k_rev;
+	tt -= rint(tt);
+	p.t0 = (float)tt;
+	p.k = k;
+	p.k2 = k * k;
+	p.ai = ai;
+}
+
+// Regular pairs of a Burton-Miller assembly under NiHu's distance-driven
+// degrees with an imaginary alpha; organised as regular_kernel.  Three of four
+// waves take bm_far, most of the others bm_mid, a few per cent bm_close.
+// 20480 triangles: 1.51 ms, 4.4 TB/s of stores; 1.32 ms without the stores,
+// 1.40 ms with the stores alone.
+template <bool MAP>
+__global__ void __launch_bounds__(256) bm_regular_kernel(RegArgs a)
+{
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
+	const int i = tile_r * 256 + threadIdx.x;
+	const bool row_ok = i < a.n_rows;
+	const int ii = row_ok ? i : a.n_rows - 1;
+	const int orow = MAP && a.rmap ? a.rmap[ii] : i;
+	const double cix = a.tc[ii], ciy = a.tc[a.tn + ii], ciz = a.tc[2 * a.tn + ii];
+	const float nxx = a.tnu[ii], nxy = a.tnu[a.tn + ii], nxz = a.tnu[2 * a.tn + ii];
+	row_ready(cix, ciy, ciz, nxx, nxy, nxz, orow);
+	const int j0 = tile_c * a.tile_cols;
+	const int j1 = min(j0 + a.tile_cols, a.n_cols);
+	const auto rec = uni(a.rec);
+	// the trial record fields of the one-point path, loaded one column ahead
+	struct Head { double cx, cy, cz, near, far; float nx, ny, nz, w1; };
+	auto head = [&](int jj) {
+		return Head{rec[jj].c[0], rec[jj].c[1], rec[jj].c[2], rec[jj].thr[THR_NEAR], rec[jj].thr[THR_22_3],
+			rec[jj].nu[0], rec[jj].nu[1], rec[jj].nu[2], rec[jj].w1};
+	};
+	Head nxt = head(j0);
+	for (int j = j0; j < j1; ++j) {
+		const Head h = nxt;
+		const double dxd = h.cx - cix, dyd = h.cy - ciy, dzd = h.cz - ciz;
+		const double d2 = __fma_rn(dzd, dzd, __fma_rn(dyd, dyd, dxd * dxd));
+		const int self = a.same_mesh ? (MAP && a.cmap ? a.cmap[j] : j) : -1;
+		const bool act = row_ok & !(d2 < h.near) & (i != self);
+		nxt = head(j + 1 < j1 ? j + 1 : j);
+		if (!any_lane(act)) continue;
+		BmPair p;
+		double d;
+		bm_geometry(dxd, dyd, dzd, d2, nxx, nxy, nxz, h.nx, h.ny, h.nz, p, d);
+		bm_wave(p, d, a.k_rev, a.k, a.alpha.y);
+		BmEntry e = {-0.0f, -0.0f, -0.0f, -0.0f};
+		if (!any_lane(act & (d2 < h.far))) {
+			bm_far(p, h.w1, e);
+		} else {
+			double t[NTHR];
+#pragma unroll
+			for (int q = 0; q < NTHR; ++q) t[q] = rec[j].thr[q];
+			if (!any_lane(act & (d2 < t[THR_3_6])))
+				bm_mid(p, nxx, nxy, nxz, a.qt[2] + (size_t)j * 3, h.w1, a.k_revf, d2 < t[THR_9_1], d2 < t[THR_15_8],
+					d2 < t[THR_22_3], e);
+			else
+				bm_close(a, j, act, d2, t, p, nxx, nxy, nxz, h.w1, a.k_revf, e);
+		}
+		if (act) {
+			const long long col = (long long)(MAP && a.cmap ? a.cmap[j] : j) * a.ld;
+			store_pair(a.out0, a.out1, col, orow, a.dtype, a.accumulate, e.ar, e.ai, e.br, e.bi);
 		}
 	}
 }
@@ -1359,8 +1600,8 @@ __device__ __forceinline__ void eval64(const Reg64Args &a, int j, int deg, D3 dc
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(256) regular64_kernel(Reg64Args a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int i = tile_r * 256 + threadIdx.x;
 	if (i >= a.n_rows) return;
 	const int orow = a.rmap ? a.rmap[i] : i;

@@ -238,8 +238,8 @@ __device__ __forceinline__ int gauss_order(int degree) { return degree / 2 + 1; 
 template <int FAM, int KM, int MODE, bool MAP, bool CK = false>
 __global__ void __launch_bounds__(256) quad_regular_kernel(QuadArgs a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int i = tile_r * 256 + threadIdx.x;
 	const bool row_ok = i < a.n_rows;
 	const int ii = row_ok ? i : a.n_rows - 1;
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256) quad_regular_kernel(QuadArgs a)
 				const int kk = (KM & SLP) ? 0 : (KM & DLP) ? 1 : (KM & DLPT) ? 2 : 3;
 				const float re = a.alpha.x * K[kk].x - a.alpha.y * K[kk].y;
 				const float im = a.alpha.x * K[kk].y + a.alpha.y * K[kk].x;
-				store_entry(a.out0, col + orow, a.dtype, a.accumulate, re, im);
+				store_row(a.out0, col, orow, a.dtype, a.accumulate, re, im);
 			} else {
 				const float ar = a.alpha.x * K[3].x - a.alpha.y * K[3].y + K[1].x;
 				const float ai = a.alpha.x * K[3].y + a.alpha.y * K[3].x + K[1].y;
@@ -715,8 +715,8 @@ __device__ __forceinline__ void quad_eval64(const Quad64Args &a, int j, int n, D
 template <int FAM, int KM, int MODE, bool CK = false>
 __global__ void __launch_bounds__(256) quad_regular64_kernel(Quad64Args a)
 {
-	const int tile_r = blockIdx.x % a.row_tiles;
-	const int tile_c = blockIdx.x / a.row_tiles;
+	int tile_r, tile_c;
+	tile_of_block(a.row_tiles, tile_r, tile_c);
 	const int i = tile_r * 256 + threadIdx.x;
 	if (i >= a.n_rows) return;
 	const int orow = a.rmap ? a.rmap[i] : i;
