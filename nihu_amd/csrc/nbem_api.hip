@@ -595,7 +595,7 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 		nbk::ListArgs a;
 		a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = same;
 		a.row_tiles = (test->n + 255) / 256;
-		a.chunk = 1024;
+		a.chunk = 128;
 		a.n_chunks = (trial->n + a.chunk - 1) / a.chunk;
 		a.tn = test->n; a.sn = trial->n;
 		a.tc = (const double *)test->d_c.get();

@@ -298,10 +298,20 @@ __device__ __forceinline__ void gal_eval_dynamic(const GalArgs &a, int e, int f,
 		const unsigned long long msel = __ballot(deg == dsel);
 		if ((msel >> __lane_id()) & 1ull) {
 			const int nq = a.qn[dsel];
-			const float *tq = (const float *)(a.tq[dsel] + (size_t)e * nq);
-			auto tp = [&](int p) { return GTest{tq[8 * p], tq[8 * p + 1], tq[8 * p + 2], tq[8 * p + 4], tq[8 * p + 7]}; };
-			gal_points<FAM, KM, NDOF, 0, decltype(tp), CK>(tp, a.sq[dsel] + (size_t)f * nq, a.ref + dsel * REF_MAXQ, nq,
-				P, a.k_revf, a.k, blk, a.ki);
+			const float4 *tq = (const float4 *)(a.tq[dsel] + (size_t)e * nq);
+			auto tp = [&](int p) {
+				const float4 t0 = tq[2 * p], t1 = tq[2 * p + 1];
+				return GTest{t0.x, t0.y, t0.z, t1.x, t1.w};
+			};
+			// the rule next to the lowest (3 or 4 points) takes most of these
+			// pairs: unrolled, its loads leave together
+			constexpr int NLOW = NDOF == 3 ? 4 : 3;
+			if (nq == NLOW)
+				gal_points<FAM, KM, NDOF, NLOW, decltype(tp), CK>(tp, a.sq[dsel] + (size_t)f * nq, a.ref + dsel * REF_MAXQ,
+					nq, P, a.k_revf, a.k, blk, a.ki);
+			else
+				gal_points<FAM, KM, NDOF, 0, decltype(tp), CK>(tp, a.sq[dsel] + (size_t)f * nq, a.ref + dsel * REF_MAXQ,
+					nq, P, a.k_revf, a.k, blk, a.ki);
 			deg = -1;
 		}
 	}
@@ -641,6 +651,35 @@ __device__ __forceinline__ float wave_sum63(float v)
 	return v;
 }
 
+// The ND x ND entries of a pair (v(x, y): valid in lane 63 as wave_sum63 leaves
+// them) change to lanes 2 (ND x + y) and that + 1 (real, imaginary part), which
+// add them to the result with one atomic instruction.
+template <int ND, class V>
+__device__ __forceinline__ void near_add(V v, const int *t_dof, int tn, int e, const int *s_dof, int sn, int f, void *out,
+	long long ld, int dtype)
+{
+	const int lane = threadIdx.x & 63;
+	int part = 0;
+#pragma unroll
+	for (int x = 0; x < ND; ++x)
+#pragma unroll
+		for (int y = 0; y < ND; ++y) {
+			const float2 t = v(x, y);
+			const int at = 2 * (ND * x + y);
+			const int re = __builtin_amdgcn_readlane(__builtin_bit_cast(int, t.x), 63);
+			const int im = __builtin_amdgcn_readlane(__builtin_bit_cast(int, t.y), 63);
+			part = lane == at ? re : lane == at + 1 ? im : part;
+		}
+	const bool real = dtype == DT_F32 || dtype == DT_F64;
+	if (lane >= 2 * ND * ND || (real && (lane & 1))) return;
+	const int x = (lane >> 1) / ND, y = (lane >> 1) % ND;
+	const long long entry = (long long)s_dof[y * sn + f] * ld + t_dof[x * tn + e];
+	const long long idx = real ? entry : 2 * entry + (lane & 1);
+	const float value = __builtin_bit_cast(float, part);
+	if (dtype == DT_C64 || dtype == DT_F32) unsafeAtomicAdd((float *)out + idx, value);
+	else unsafeAtomicAdd((double *)out + idx, (double)value);
+}
+
 // Pairs of a near list (test, trial element) and the dofs of their corners
 struct GalNear {
 	int n_pairs;
@@ -654,7 +693,8 @@ struct GalNear {
 // one lane busy with up to 19 x 19 points while its wave waits, and the chunk
 // of trial elements next to a tile's own sets the launch's time (double layer,
 // 4332 elements: 3.66 ms; 0.73 ms with these pairs taken here and chunks of 8
-// elements).  A handful of them per element, so one atomic per entry.
+// elements; the kernel itself 389 -> 184 us since its entries go out in one
+// atomic instruction).
 template <int FAM, int KM, int NDOF, bool CK = false>
 __global__ void __launch_bounds__(256) galerkin_near_kernel(GalArgs a, GalNear l)
 {
@@ -721,19 +761,17 @@ __global__ void __launch_bounds__(256) galerkin_near_kernel(GalArgs a, GalNear l
 	// (idle lanes hold zeros)
 	const float w = sq[3], w1 = sq[5], w2 = sq[6];
 	const float wb[3] = {NDOF == 1 ? w : w - w1 - w2, w1, w2};
-#pragma unroll
-	for (int x = 0; x < NDOF; ++x)
-#pragma unroll
-		for (int y = 0; y < NDOF; ++y) {
-			const float vr = wave_sum63(T[x].x * wb[y]);
-			const float vi = FAM == HELM ? wave_sum63(T[x].y * wb[y]) : 0.0f;
-			const float re = a.alpha.x * vr - a.alpha.y * vi;
-			const float im = a.alpha.x * vi + a.alpha.y * vr;
-			if (lane != 63) continue;
-			if (NDOF == 1) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, re, im);
-			else
-				atomic_add_entry(a.out, (long long)l.s_dof[y * a.sn + f] * a.ld + l.t_dof[x * a.tn + e], a.dtype, re, im);
-		}
+	auto entry = [&](int x, int y) {
+		const float vr = wave_sum63(T[x].x * wb[y]);
+		const float vi = FAM == HELM ? wave_sum63(T[x].y * wb[y]) : 0.0f;
+		return make_float2(a.alpha.x * vr - a.alpha.y * vi, a.alpha.x * vi + a.alpha.y * vr);
+	};
+	if (NDOF == 1) {
+		const float2 v = entry(0, 0);
+		if (lane == 63) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, v.x, v.y);
+	} else {
+		near_add<NDOF>(entry, l.t_dof, a.tn, e, l.s_dof, a.sn, f, a.out, a.ld, a.dtype);
+	}
 }
 
 // ---------------------------------------------------------------- FP64 pass

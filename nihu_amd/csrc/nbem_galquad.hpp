@@ -482,19 +482,17 @@ __global__ void __launch_bounds__(256) galq_near_kernel(GalQArgs a, GalNear l)
 	// the trial weights w J N_b of the lane's point, then the sum over the
 	// lanes (idle lanes hold zeros)
 	const float wb[4] = {ND == 1 ? ((const float *)sr)[12] : s2.x, s2.y, s2.z, s2.w};
-#pragma unroll
-	for (int c = 0; c < ND; ++c)
-#pragma unroll
-		for (int b = 0; b < ND; ++b) {
-			const float vr = wave_sum63(T[c].x * wb[b]);
-			const float vi = FAM == HELM ? wave_sum63(T[c].y * wb[b]) : 0.0f;
-			const float re = a.alpha.x * vr - a.alpha.y * vi;
-			const float im = a.alpha.x * vi + a.alpha.y * vr;
-			if (lane != 63) continue;
-			if (ND == 1) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, re, im);
-			else
-				atomic_add_entry(a.out, (long long)l.s_dof[b * a.sn + f] * a.ld + l.t_dof[c * a.tn + e], a.dtype, re, im);
-		}
+	auto entry = [&](int c, int b) {
+		const float vr = wave_sum63(T[c].x * wb[b]);
+		const float vi = FAM == HELM ? wave_sum63(T[c].y * wb[b]) : 0.0f;
+		return make_float2(a.alpha.x * vr - a.alpha.y * vi, a.alpha.x * vi + a.alpha.y * vr);
+	};
+	if (ND == 1) {
+		const float2 v = entry(0, 0);
+		if (lane == 63) store_entry(a.out, (long long)f * a.ld + e, a.dtype, 1, v.x, v.y);
+	} else {
+		near_add<ND>(entry, l.t_dof, a.tn, e, l.s_dof, a.sn, f, a.out, a.ld, a.dtype);
+	}
 }
 
 struct GalQSingArgs {
@@ -555,9 +553,11 @@ __global__ void __launch_bounds__(64) galq_singular_kernel(GalQSingArgs a)
 		quad_dx(Qt, txi, teta, a1, b1);
 		quad_dx(Qs, sxi, seta, a2, b2);
 		const D3 n1 = d3cross(a1, b1), n2 = d3cross(a2, b2);
-		const double J1 = d3norm(n1), J2 = d3norm(n2);
+		const double s1 = d3dot(n1, n1), s2 = d3dot(n2, n2);
+		const double i1 = rsqrt64(s1), i2 = rsqrt64(s2);
+		const double J1 = s1 * i1, J2 = s2 * i2;
 		const D3 x = quad_x(Qt, txi, teta), y = quad_x(Qs, sxi, seta);
-		const D3 u1 = d3scale(n1, ot / J1), u2 = d3scale(n2, os / J2);
+		const D3 u1 = d3scale(n1, ot * i1), u2 = d3scale(n2, os * i2);
 		const double2 K = CK ? kernel_value64_c<KM>(x, y, u1, u2, a.k, a.ki) : kernel_value64<FAM, KM>(x, y, u1, u2, a.k);
 		const double wt = J1 * w, ws = J2;
 		if (ND == 1) {

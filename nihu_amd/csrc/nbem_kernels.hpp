@@ -1707,6 +1707,10 @@ __device__ __forceinline__ bool list_share_node(const ListArgs &a, int i, int j)
 	return false;
 }
 
+// One row per lane, a chunk of columns per workgroup; the trial side comes
+// through the scalar cache, four columns at a time.  Bound by the chain of a
+// chunk's columns: with 128 columns instead of 1024 and without a vector load
+// per column, 8192 x 3456 pairs: count 146 -> 17 us, fill 106 -> 15 us.
 template <bool FILL>
 __global__ void __launch_bounds__(256) near_list_kernel(ListArgs a)
 {
@@ -1716,15 +1720,28 @@ __global__ void __launch_bounds__(256) near_list_kernel(ListArgs a)
 	if (i >= a.n_rows) return;
 	const double cix = a.tc[i], ciy = a.tc[a.tn + i], ciz = a.tc[2 * a.tn + i];
 	const int j0 = ch * a.chunk, j1 = min(j0 + a.chunk, a.n_cols);
+	const auto sc = uni(a.sc), thr = uni(a.thr_near);
 	int cnt = 0;
-	int base = FILL ? a.offsets[(long long)i * a.n_chunks + ch] : 0;
-	for (int j = j0; j < j1; ++j) {
-		const double d2 = d2_pair(cix, ciy, ciz, a.sc[j], a.sc[a.sn + j], a.sc[2 * a.sn + j]);
-		if (d2 < a.thr_near[j] && !(a.same_mesh && i == j) && !(a.t_node && list_share_node(a, i, j))) {
+	const int base = FILL ? a.offsets[(long long)i * a.n_chunks + ch] : 0;
+	auto column = [&](int j, double d2, double lim) {
+		if (d2 < lim && !(a.same_mesh && i == j) && !(a.t_node && list_share_node(a, i, j))) {
 			if (FILL) { a.pi[base + cnt] = i; a.pj[base + cnt] = j; }
 			++cnt;
 		}
+	};
+	int j = j0;
+	for (; j + 4 <= j1; j += 4) {
+		double d2[4], lim[4];
+#pragma unroll
+		for (int u = 0; u < 4; ++u) {
+			d2[u] = d2_pair(cix, ciy, ciz, sc[j + u], sc[a.sn + j + u], sc[2 * a.sn + j + u]);
+			lim[u] = thr[j + u];
+		}
+		if (!any_lane((d2[0] < lim[0]) | (d2[1] < lim[1]) | (d2[2] < lim[2]) | (d2[3] < lim[3]))) continue;
+#pragma unroll
+		for (int u = 0; u < 4; ++u) column(j + u, d2[u], lim[u]);
 	}
+	for (; j < j1; ++j) column(j, d2_pair(cix, ciy, ciz, sc[j], sc[a.sn + j], sc[2 * a.sn + j]), thr[j]);
 	if (!FILL) a.counts[(long long)i * a.n_chunks + ch] = cnt;
 }
 
