@@ -373,7 +373,7 @@ struct nb_mesh {
 	// field in a pair with a nodal one)
 	struct GalLayout {
 		int tiles = 0, chunk = 0;
-		DevPtr elem, contrib, rows, fin;
+		DevPtr elem, contrib, rows, fin, first;
 	} glay[2];
 	// Galerkin trial sequences: in the order of glay[0], glay[1], element order
 	DevPtr d_grec[3];
@@ -779,9 +779,16 @@ int ensure_gal_layout(nb_mesh *m, int kind = 0)
 	if (nbg_galerkin_layout_n(n, dm.data(), npe, cs, m->c.data(), chunk, order.data(), elem.data(),
 		contrib.data(), rows.data(), col.data(), fin.data()) != tiles)
 		return fail(NB_ERR_RUNTIME, "Galerkin layout");
+	// sequence position of each tile's first element (tiles hold consecutive ones)
+	std::vector<int32_t> first(tiles, 0);
+	for (int t = 1; t < tiles; ++t) {
+		int cnt = 0;
+		for (int l = 0; l < nbk::GAL_TILE; ++l) cnt += elem[(size_t)(t - 1) * nbk::GAL_TILE + l] >= 0;
+		first[t] = first[t - 1] + cnt;
+	}
 	int s;
 	if ((s = upload(L.elem, elem)) || (s = upload(L.contrib, contrib)) || (s = upload(L.rows, rows)) ||
-		(s = upload(L.fin, fin)) || (s = upload_gal_rec(m, kind, order.data(), col.data())))
+		(s = upload(L.fin, fin)) || (s = upload(L.first, first)) || (s = upload_gal_rec(m, kind, order.data(), col.data())))
 		return s;
 	L.tiles = tiles;
 	L.chunk = chunk;
@@ -1161,6 +1168,7 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		a.t_elem = (const int *)test->glay[kt].elem.get();
 		a.t_contrib = (const uint2 *)test->glay[kt].contrib.get();
 		a.t_rows = (const int *)test->glay[kt].rows.get();
+		a.t_first = (const int *)test->glay[kt].first.get();
 		a.rec = (const nbk::GalRec *)trial->d_grec[ks].get();
 		a.s_fin = (const int *)trial->glay[ks].fin.get();
 	} else {
@@ -1169,6 +1177,11 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		if (!trial->d_grec[2] && (s = upload_gal_rec(trial, 2, nullptr, nullptr))) return s;
 		a.rec = (const nbk::GalRec *)trial->d_grec[2].get();
 	}
+	// one mesh, one fixed rule, nodal fields on both sides, the single layer: each
+	// pair of elements once, its mirror image by symmetrise_kernel -- for a result
+	// that starts from zero (what an accumulated one holds must not be mirrored)
+	const bool sym = jb.same && jb.km == nbk::SLP && lt && ls && jb.pol.rule == NB_RULE_FIXED && !accumulate;
+	a.sym = sym ? 1 : 0;
 	a.tn = test->n; a.sn = trial->n; a.same_mesh = jb.same;
 	a.t_tri = (const int *)test->d_tri.get();
 	a.tc = (const double *)test->d_c.get();
@@ -1250,6 +1263,18 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 #undef NB_GALN
 		}
 		NB_HIP(hipGetLastError());
+		if (sym) {
+			const long long nb = (rows + 31) / 32, pairs = nb * (nb + 1) / 2;
+			if (pairs > 0x7fffffffLL) return fail(NB_ERR_RANGE, "matrix too large");
+			const dim3 g((unsigned)pairs), w(256);
+			switch (dtype) {
+			case NB_C64: hipLaunchKernelGGL((symmetrise_kernel<float2>), g, w, 0, st, (float2 *)out, (long long)ld, (int)rows); break;
+			case NB_C128: hipLaunchKernelGGL((symmetrise_kernel<double2>), g, w, 0, st, (double2 *)out, (long long)ld, (int)rows); break;
+			case NB_F32: hipLaunchKernelGGL((symmetrise_kernel<float>), g, w, 0, st, (float *)out, (long long)ld, (int)rows); break;
+			default: hipLaunchKernelGGL((symmetrise_kernel<double>), g, w, 0, st, (double *)out, (long long)ld, (int)rows); break;
+			}
+			NB_HIP(hipGetLastError());
+		}
 		prof_end(pe, st);
 	}
 	if (!jb.same) return NB_OK;

@@ -112,3 +112,51 @@ def test_galerkin_mostly_close_pairs(nb, quads):
     whole, part = nb.Mesh(nodes, el), nb.Mesh(nodes, np.ascontiguousarray(el[:2000]))
     for ny in (0, 1):
         check(galerkin(nb, part, t, "galerkin", ny, 2.0), galerkin(nb, whole, t, "galerkin", ny, 2.0)[:2000])
+
+
+@pytest.mark.parametrize("kind", [("complex64", False), ("complex64", True), ("complex128", False)],
+                         ids=["c64", "c64-accumulate", "c128"])
+@pytest.mark.parametrize("degree", [4, 2])
+@pytest.mark.parametrize("n_elem", [1, 2, 63, 65, 129, 701])
+def test_galerkin_fixed_single_layer(nb, orc, n_elem, degree, kind):
+    # one mesh, one rule: pairs taken once and mirrored (not into a result that
+    # already holds something)
+    import torch
+    nodes, el = surface(n_elem)
+    m = nb.Mesh(nodes, el)
+    n = m.n_nodes
+    rng = np.random.default_rng(n_elem)
+    ref = orc.assemble_galerkin(nodes, el, 1, 0, 0, k=3.0, linear=True, pol=orc.policy(rule=1, fixed_degree=degree))
+    out = nb.colmajor(n, n, kind[0])
+    old = np.zeros((n, n), dtype=complex)
+    if kind[1]:
+        old = (rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))) * np.abs(ref).max()
+        out.copy_(torch.from_numpy(old))
+    nb.assemble(m, m, out, nb.NB_HELMHOLTZ, 0, 0, 3.0, pol=nb.policy("fixed", degree=degree), accumulate=kind[1],
+                formalism="galerkin_linear")
+    torch.cuda.synchronize()
+    # an accumulated float32 entry also rounds the old content (up to 5 times the largest entry)
+    assert np.abs(out.cpu().numpy() - old - ref).max() < 2e-6 * np.abs(ref).max()
+
+
+def test_field_blocks_follow_the_arrays(nb):
+    # more field points than one block: the kept blocks give the result of a new
+    # mesh, also after the field mesh's node array has changed
+    import torch
+    from nihu_amd import postproc
+    from nihu_amd.mesh import create_slab
+    nodes, quads = surface(54, quads=True)
+    s = nb.Mesh(nodes, quads)
+    corners = np.array([[-2, -2, 2.5], [2, -2, 2.5], [2, 2, 3], [-2, 2, 3]], dtype=float)
+    fn, fe = create_slab(corners, 20, 15)
+    field = nb.Mesh(fn, fe)
+    p = torch.ones(54, dtype=torch.complex128, device="cuda")
+    first = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=128)
+    again = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=128)
+    whole = postproc.field_pressure(field, s, 2.0, p, 1j * p)
+    assert torch.equal(first, again)
+    assert (first - whole).abs().max() <= 1e-12 * whole.abs().max()
+    field.nodes[:, 2] += 0.5
+    moved = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=128)
+    fresh = postproc.field_pressure(nb.Mesh(field.nodes.copy(), fe), s, 2.0, p, 1j * p, block_rows=128)
+    assert torch.equal(moved, fresh)
