@@ -3068,7 +3068,9 @@ int nb_gemv_c64(const void *A, int64_t rows, int64_t cols, int64_t ld, const voi
 	if (blocks > 0x7fffffffLL) return fail(NB_ERR_RANGE, "matrix too large");
 	g.A = (const float2 *)A; g.rows = rows; g.cols = cols; g.ld = ld;
 	g.x = (const double2 *)x; g.y = (double2 *)y; g.work = (double2 *)work;
-	hipLaunchKernelGGL(nbk::gemv_partial_kernel, dim3((unsigned)blocks), dim3(256), 0, st, g);
+	// matrices of 512 MB and more stream past the caches
+	if (rows * cols >= (1ll << 26)) hipLaunchKernelGGL(nbk::gemv_partial_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, g);
+	else hipLaunchKernelGGL(nbk::gemv_partial_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, g);
 	NB_HIP(hipGetLastError());
 	hipLaunchKernelGGL(nbk::gemv_reduce_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, st, g);
 	NB_HIP(hipGetLastError());

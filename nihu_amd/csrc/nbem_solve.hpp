@@ -30,6 +30,11 @@ struct GemvArgs {
 	long long clen;     // columns per chunk
 };
 
+// STREAM: a matrix that does not fit the 256 MB memory-side cache is read
+// non-temporally (20480 square: 570 -> 531 us a product, 6.3 TB/s; 10000: 156 ->
+// 141), a smaller one may stay there from product to product (6000: 53 us plain,
+// 56 non-temporal; 5120: 38 and 41).
+template <bool STREAM>
 __global__ void __launch_bounds__(256) gemv_partial_kernel(GemvArgs a)
 {
 	const int tile = blockIdx.x % a.row_tiles;
@@ -40,13 +45,18 @@ __global__ void __launch_bounds__(256) gemv_partial_kernel(GemvArgs a)
 	const long long j0 = (long long)ch * a.clen;
 	const long long j1 = min(j0 + a.clen, a.cols);
 	const auto x = uni((const double *)a.x);   // x[2 j], x[2 j + 1]: re, im of x_j
+	typedef float V __attribute__((ext_vector_type(2)));
 	double re = 0.0, im = 0.0;
 	long long j = j0;
 	// eight columns per step: eight independent loads in flight per lane
 	for (; j + 8 <= j1; j += 8) {
 		float2 v[8];
 #pragma unroll
-		for (int u = 0; u < 8; ++u) v[u] = a.A[(j + u) * a.ld + ii];
+		for (int u = 0; u < 8; ++u) {
+			const V *p = (const V *)a.A + ((j + u) * a.ld + ii);
+			const V t = STREAM ? __builtin_nontemporal_load(p) : *p;
+			v[u] = make_float2(t.x, t.y);
+		}
 #pragma unroll
 		for (int u = 0; u < 8; ++u) {
 			const double xr = x[2 * (j + u)], xi = x[2 * (j + u) + 1];
@@ -70,7 +80,17 @@ __global__ void __launch_bounds__(256) gemv_reduce_kernel(GemvArgs a)
 	const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
 	if (i >= a.rows) return;
 	double re = 0.0, im = 0.0;
-	for (int c = 0; c < a.chunks; ++c) {
+	// eight loads in flight, the sum in order (300 x 20480, 320 chunks a row: 92 ->
+	// 28 us a product)
+	int c = 0;
+	for (; c + 8 <= a.chunks; c += 8) {
+		double2 v[8];
+#pragma unroll
+		for (int u = 0; u < 8; ++u) v[u] = a.work[(long long)(c + u) * a.rows + i];
+#pragma unroll
+		for (int u = 0; u < 8; ++u) { re += v[u].x; im += v[u].y; }
+	}
+	for (; c < a.chunks; ++c) {
 		const double2 v = a.work[(long long)c * a.rows + i];
 		re += v.x;
 		im += v.y;

@@ -160,3 +160,23 @@ def test_field_blocks_follow_the_arrays(nb):
     moved = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=128)
     fresh = postproc.field_pressure(nb.Mesh(field.nodes.copy(), fe), s, 2.0, p, 1j * p, block_rows=128)
     assert torch.equal(moved, fresh)
+
+
+@pytest.mark.parametrize("rows,cols,ld", [(1, 5, 1), (257, 3001, 300), (8191, 8193, 8191), (8192, 8192, 8192),
+                                          (8195, 8195, 8201)])
+def test_product_sizes(nb, rows, cols, ld):
+    """Matrix-vector product on both sides of the size from which the matrix
+    is read past the caches, with partial steps of eight columns and chunks and a
+    padded leading dimension; bound of FP64 sums in any order, cols * 2^-52 times
+    sum |a| |x|."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    A = torch.randn(cols, ld, dtype=torch.complex64, device="cuda", generator=g).t()[:rows]
+    x = torch.randn(cols, dtype=torch.complex128, device="cuda", generator=g)
+    y = nb.gemv(A, x)
+    ref, mag = torch.zeros_like(y), torch.zeros(rows, dtype=torch.float64, device="cuda")
+    for j in range(0, cols, 1024):
+        b = A[:, j:j + 1024].to(torch.complex128)
+        ref += (b * x[j:j + 1024]).sum(1)
+        mag += (b.abs() * x[j:j + 1024].abs()).sum(1)
+    assert ((y - ref).abs() <= cols * 2.0 ** -52 * mag).all()
