@@ -239,17 +239,18 @@ class Mesh:
         check(lib().nb_mesh_info(self._h, None, None, C.byref(b)))
         return b.value
 
-    def block(self, r0, r1):
-        """The mesh of this mesh's elements r0 .. r1 - 1, kept until this mesh is
-        closed (the latest 32).  A block is built again when the arrays no longer
+    def block(self, r0, r1, device=0):
+        """The mesh of this mesh's elements r0 .. r1 - 1 on the current device
+        (number `device`: a mesh lives where it was created), kept until this mesh
+        is closed (the latest 32).  A block is built again when the arrays no longer
         hold what it was built from."""
         blocks = self.__dict__.setdefault("_blocks", {})
-        sub = blocks.get((r0, r1))
+        sub = blocks.get((device, r0, r1))
         if sub is None or not (np.array_equal(sub.nodes, self.nodes) and np.array_equal(sub.tris, self.tris[r0:r1])):
             sub = Mesh(self.nodes.copy(), self.tris[r0:r1].copy())
             while len(blocks) >= 32:
                 blocks.pop(next(iter(blocks)), None)
-            blocks[(r0, r1)] = sub
+            blocks[(device, r0, r1)] = sub
         return sub
 
     def close(self):

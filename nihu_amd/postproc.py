@@ -50,7 +50,7 @@ def field_pressure(field: "nbem.Mesh", surface: "nbem.Mesh", k: float, p, q, pol
     # included, took half of a repeated call's 1.85 ms)
     for r0 in range(0, m, block_rows):
         r1 = min(m, r0 + block_rows)
-        sub = field if (r0 == 0 and r1 == m) else field.block(r0, r1)
+        sub = field if (r0 == 0 and r1 == m) else field.block(r0, r1, torch.cuda.current_device())
         L = nbem.colmajor(r1 - r0, n, dtype)
         M = nbem.colmajor(r1 - r0, n, dtype)
         nbem.assemble(sub, surface, L, nbem.NB_HELMHOLTZ, 0, 0, k, pol=pol, same_mesh=False, accumulate=False)
