@@ -649,7 +649,7 @@ __global__ void __launch_bounds__(256) galerkin_regular_kernel(GalArgs a)
 // 2 for nb tiles a side).  The regular single-layer pairs of one mesh under one
 // fixed rule are symmetric (the kernel is, and both elements carry the same
 // rule), so the regular pass takes each pair of elements once and this pass
-// adds the mirror images: 10242 nodes, 6 x 6 points: 12.8 -> 6.9 ms with it.
+// adds the mirror images: 10242 nodes, 6 x 6 points: 12.8 -> 8.1 ms with it.
 template <class T>
 __global__ void __launch_bounds__(256) symmetrise_kernel(T *out, long long ld, int n)
 {
