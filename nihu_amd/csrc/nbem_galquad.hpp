@@ -217,7 +217,9 @@ struct GalqTest2 { float ax, ay, az, aa, nx, ny, nz, w; };
 // and h- = (1 - 1/sqrt 3)/2 per axis, so the sums with N_b over the points are
 // two stages of h+ (v + rho v') and h+ (rho v + v'), rho = h-/h+ = 2 - sqrt 3:
 // 8 FMAs instead of 16 for the four sums of a real part; the four factors h+
-// ride on the test weights.  Replaces blk.
+// ride on the test weights, which the point rows hold with them (column 13,
+// formed in FP64 and rounded once: with an FP32 factor h+^4, 2.6e-8 too small
+// for every entry, the matrices had 6 to 15 % more error).  Replaces blk.
 template <int FAM, int KM, bool CK>
 __device__ __forceinline__ void galq_two(const GalqTest2 (&t)[4], const float *sq_in, const GalPair &P, float k_revf, float k,
 	float2 (&blk)[4][4], float kim)
@@ -313,12 +315,10 @@ __global__ void __launch_bounds__(256) galq_regular_kernel(GalQArgs a)
 	if (a.fixed_n <= 0) {
 		const int nq = ND == 4 ? 4 : 1;
 		const float *tp = a.tq[ND == 4 ? 2 : 1] + (size_t)ee * nq * GALQ_ROW;
-		// h+^4, h+ = (1 + 1 / sqrt 3) / 2
-		const float scale = ND == 4 ? 0.38689453417431970f : 1.0f;
 #pragma unroll
 		for (int p = 0; p < nq; ++p) {
 			const float4 t0 = *(const float4 *)(tp + GALQ_ROW * p), t1 = *(const float4 *)(tp + GALQ_ROW * p + 4);
-			tp2[p] = GalqTest2{t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, scale * tp[GALQ_ROW * p + 12]};
+			tp2[p] = GalqTest2{t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, tp[GALQ_ROW * p + (ND == 4 ? 13 : 12)]};
 		}
 		if (ND == 1) { P.nxx = tp2[0].nx; P.nxy = tp2[0].ny; P.nxz = tp2[0].nz; }
 	}

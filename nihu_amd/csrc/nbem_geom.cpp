@@ -389,10 +389,14 @@ int nbg_quad4_table(int N, int n, const double *c, const double *X, float *out)
 // Gauss square rule with N x N points (xi outer, eta inner) for the Galerkin
 // passes on quadrilaterals: out[(e * N*N + q) * 16 + {0..15}] =
 // o = y_q - c_e (xyz), |o|^2, unit normal n at y_q (xyz), o.n,
-// w_q J(xi_q) N_b(xi_q) for the four corners b, w_q J(xi_q), 0, 0, 0 (floats).
+// w_q J(xi_q) N_b(xi_q) for the four corners b, w_q J(xi_q), w_q J(xi_q) h^4,
+// 0, 0 (floats).  h = (1 + 1/sqrt 3) / 2, the larger shape function per axis at
+// the points of the 2 x 2 rule, as 1 / (1 + rho) of the FP32 rho = 2 - sqrt 3 that
+// rule is evaluated with (galq_two), so that the shape functions sum to 1.
 int nbg_quad_gal_table(int N, int n, const double *c, const double *X, float *out)
 {
 	if (N < 1 || N > 64) return -1;
+	const double h = 1.0 / (1.0 + (double)0.26794919243112270647f), h4 = h * h * h * h;
 	std::vector<double> gx(N), gw(N);
 	nbg_gauss_legendre(N, gx.data(), gw.data());
 	for (int e = 0; e < n; ++e) {
@@ -417,7 +421,8 @@ int nbg_quad_gal_table(int N, int n, const double *c, const double *X, float *ou
 				p[7] = (float)(o.x * u.x + o.y * u.y + o.z * u.z);
 				for (int b = 0; b < 4; ++b) p[8 + b] = (float)(w * N4[b]);
 				p[12] = (float)w;
-				p[13] = p[14] = p[15] = 0.0f;
+				p[13] = (float)(w * h4);
+				p[14] = p[15] = 0.0f;
 			}
 	}
 	return N * N;
