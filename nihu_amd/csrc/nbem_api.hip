@@ -113,6 +113,7 @@ int upload(DevPtr &p, const std::vector<T> &v)
 
 struct NearList {
 	uint64_t test_uid;
+	std::weak_ptr<char> test_alive;   // expired once the test mesh is destroyed
 	int same, mode;
 	double limit;
 	int n;
@@ -363,9 +364,10 @@ struct nb_mesh {
 	DevPtr d_qt64[nbk::NSLOT];      // FP64 point tables of the FP64 precision policy
 	DevPtr d_qq[nbk::QN_MAX + 1];              // quadrilaterals: Gauss square tables by order
 	DevPtr d_qq64[nbk::QN_MAX + 1];            // the same in FP64 (y, w J, unit normal): FP64 precision policy
-	// near-pair lists per (test mesh, near policy), oldest first; callers hold
-	// a list by shared_ptr, so evicting it cannot free one in use
+	// near-pair lists per (test mesh, near policy), least recently used first;
+	// callers hold a list by shared_ptr, so evicting it cannot free one in use
 	std::vector<std::shared_ptr<NearList> > near_cache;
+	std::shared_ptr<char> alive = std::make_shared<char>();   // the lists of other meshes watch it
 	std::vector<int32_t> tri;                  // element-major node ids (host)
 	DevPtr d_tri;                              // node ids [npe][n] (quadrilaterals: uploaded on first use)
 	// Galerkin, nodal dofs: element order, wave tiles, column-slot schedule
@@ -567,19 +569,53 @@ void policy_degrees(const nb_policy &p, int km, int field_complexity, std::vecto
 	deg.erase(std::unique(deg.begin(), deg.end()), deg.end());
 }
 
-// the cached list of (test mesh, near policy), or null
-std::shared_ptr<NearList> find_near_list(const nb_mesh *trial, const nb_mesh *test, int same, const nb_policy &pol)
-{
-	for (auto &nl : trial->near_cache)
-		if (nl->test_uid == test->uid && nl->same == same && nl->mode == pol.near_mode && nl->limit == pol.near_limit)
-			return nl;
-	return nullptr;
-}
-
 // Near-pair lists.  slot THR_NEAR: the near-singular pairs of a policy.
 // Another slot: the pairs of the Galerkin formalism inside that breakpoint of
 // the distance tables that share no node (kept under the mode GAL_LIST + slot).
 constexpr int GAL_LIST = 64;
+
+// the cached list of (test mesh, near policy), or null
+std::shared_ptr<NearList> find_near_list(nb_mesh *trial, const nb_mesh *test, int same, const nb_policy &pol)
+{
+	auto &c = trial->near_cache;
+	for (size_t i = 0; i < c.size(); ++i)
+		if (c[i]->test_uid == test->uid && c[i]->same == same && c[i]->mode == pol.near_mode &&
+			c[i]->limit == pol.near_limit) {
+			std::rotate(c.begin() + i, c.begin() + i + 1, c.end());   // now the latest used
+			return c.back();
+		}
+	return nullptr;
+}
+
+// Lists of one kind do not displace those of another: 0 the mesh's own
+// near-singular lists (the allocation-free sweep needs its one resident), 1
+// those against other test meshes, 2 the Galerkin formalism's.
+int near_list_kind(const NearList &nl) { return nl.mode >= GAL_LIST ? 2 : nl.same ? 0 : 1; }
+
+// Keep a list: those whose test mesh is gone leave, then the least recently
+// used of its kind beyond 8 -- of those against other test meshes beyond 64
+// while they hold less than 256 MB together (a caller that goes round its test
+// meshes, the blocks of a field mesh among them, finds them all again).
+void keep_near_list(nb_mesh *trial, const std::shared_ptr<NearList> &nl)
+{
+	auto &c = trial->near_cache;
+	const int kind = near_list_kind(*nl);
+	int count = 1;
+	int64_t bytes = (int64_t)nl->n * 8;
+	for (auto &q : c)
+		if (near_list_kind(*q) == kind && !q->test_alive.expired()) { ++count; bytes += (int64_t)q->n * 8; }
+	for (size_t i = 0; i < c.size();) {
+		const bool gone = c[i]->test_alive.expired();
+		const bool over = near_list_kind(*c[i]) == kind && count > 8 && (kind == 0 || count > 64 || bytes > (256ll << 20));
+		if (!gone && !over) { ++i; continue; }
+		const int64_t b = (int64_t)c[i]->n * 8;
+		if (!gone) { --count; bytes -= b; }
+		trial->bytes -= b;
+		c.erase(c.begin() + i);
+	}
+	trial->bytes += (int64_t)nl->n * 8;
+	c.push_back(nl);
+}
 
 int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy pol, hipStream_t st,
 	std::shared_ptr<NearList> *out, int slot = nbk::THR_NEAR)
@@ -590,7 +626,8 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 	}
 	if ((*out = find_near_list(trial, test, same, pol))) return NB_OK;
 	std::shared_ptr<NearList> nl(new NearList());
-	nl->test_uid = test->uid; nl->same = same; nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0;
+	nl->test_uid = test->uid; nl->test_alive = test->alive; nl->same = same;
+	nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0;
 	if (pol.near_mode != NB_NEAR_NONE) {
 		nbk::ListArgs a;
 		a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = same;
@@ -632,13 +669,8 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 		hipLaunchKernelGGL(nbk::near_list_kernel<true>, dim3(grid), dim3(256), 0, st, a);
 		NB_HIP(hipGetLastError());
 		NB_HIP(hipStreamSynchronize(st));   // counts/offsets are freed on return
-		trial->bytes += (int64_t)nl->n * 8;
 	}
-	if (trial->near_cache.size() >= 8) {
-		trial->bytes -= (int64_t)trial->near_cache.front()->n * 8;
-		trial->near_cache.erase(trial->near_cache.begin());
-	}
-	trial->near_cache.push_back(nl);
+	keep_near_list(trial, nl);
 	*out = std::move(nl);
 	return NB_OK;
 }

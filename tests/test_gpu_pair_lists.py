@@ -1,0 +1,79 @@
+"""The kept lists of close pairs: what displaces what, what they hold of device
+memory (8 bytes per listed pair, in the trial mesh's byte count), and what a
+call does that has none."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nb():
+    import torch
+    assert torch.cuda.is_available(), "GPU test without a GPU"
+    from nihu_amd import nbem
+    return nbem
+
+
+def sphere(level=2, move=0.0, seed=0):
+    from nihu_amd.mesh import jittered_icosphere
+    nodes, tris = jittered_icosphere(level, seed=seed)
+    return nodes + np.array([move, 0.0, 0.0]), tris
+
+
+def operator(nb, test, trial, form, ny=0, pol=None, dtype="complex64"):
+    import torch
+    out = nb.colmajor(test.dofs(form, "test"), trial.dofs(form, "trial"), dtype)
+    nb.assemble(test, trial, out, nb.NB_HELMHOLTZ, 0, ny, 3.0, pol=pol, accumulate=False, formalism=form)
+    torch.cuda.synchronize()
+    return out
+
+
+def test_other_lists_leave_the_sweeps_resident(nb):
+    # Galerkin calls and collocation against other meshes, more than eight of
+    # each: the mesh's own near list, which the allocation-free sweep takes, stays
+    import torch
+    m = nb.Mesh(*sphere())
+    ks = np.array([2.0, 3.0])
+    A, B = (torch.zeros((2, m.n, m.n), dtype=torch.complex64, device="cuda").transpose(1, 2) for _ in range(2))
+    nb.assemble_sweep(m, ks, A, B)
+    want = A.clone(), B.clone()
+    others = [nb.Mesh(*sphere(1, 0.1 * i)) for i in range(5)]
+    for t in others:
+        for ny in (0, 1):
+            operator(nb, t, m, "galerkin_linear", ny)
+            operator(nb, t, m, "collocation", ny, nb.policy("nihu", limit=1.5 + 0.01 * ny))
+    # the sweep's own thresholds again: the last policy above had others
+    operator(nb, others[0], m, "collocation", 0, nb.policy("nihu"))
+    nb.assemble_sweep(m, ks, A, B, noalloc=True)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.view_as_real(A), torch.view_as_real(want[0]))
+    assert torch.equal(torch.view_as_real(B), torch.view_as_real(want[1]))
+
+
+@pytest.mark.parametrize("form", ["collocation", "galerkin"])
+def test_lists_of_many_test_meshes(nb, form):
+    # twelve test meshes in turn: all their lists stay (a second round builds
+    # nothing), and leave once their mesh is gone
+    m = nb.Mesh(*sphere())
+    tests = [nb.Mesh(*sphere(1, 0.05 * i)) for i in range(12)]
+    operator(nb, tests[0], m, form)          # tables
+    base, seen = m.device_bytes(), []
+    for t in tests[1:]:
+        operator(nb, t, m, form)
+        seen.append(m.device_bytes())
+    grown = np.diff([base] + seen)
+    assert (grown >= 0).all() and grown.sum() > 0
+    for t in tests:
+        operator(nb, t, m, form)
+        assert m.device_bytes() == seen[-1]
+    tests.clear()
+    del t
+    operator(nb, m, m, form)
+    own = m.device_bytes()
+    operator(nb, nb.Mesh(*sphere(1, 40.0)), m, form)      # far away: an empty list
+    assert m.device_bytes() == own
+    fresh = nb.Mesh(*sphere())
+    operator(nb, fresh, fresh, form)
+    assert own == fresh.device_bytes()
