@@ -117,6 +117,7 @@ struct NearList {
 	int same, mode;
 	double limit;
 	int n;
+	bool refused;                     // more pairs than the caller takes as a list: none are held
 	DevPtr pi, pj;
 };
 
@@ -569,6 +570,18 @@ void policy_degrees(const nb_policy &p, int km, int field_complexity, std::vecto
 	deg.erase(std::unique(deg.begin(), deg.end()), deg.end());
 }
 
+// zero_kernel over a rows x cols block: one grid row per column (up to 65535,
+// the kernel strides beyond), enough blocks along x for a column of 16-byte words
+void launch_zero(void *out, int64_t ld, int64_t rows, int64_t cols, int elem_bytes, hipStream_t st)
+{
+	if (rows <= 0 || cols <= 0) return;
+	const int64_t words16 = (rows * elem_bytes + 15) / 16;
+	const unsigned gx = (unsigned)std::min<int64_t>((words16 + 255) / 256, 64);
+	const unsigned gy = (unsigned)std::min<int64_t>(cols, 65535);
+	hipLaunchKernelGGL(nbk::zero_kernel, dim3(gx, gy), dim3(256), 0, st, out, (long long)ld, (long long)rows,
+		(long long)cols, elem_bytes);
+}
+
 // Near-pair lists.  slot THR_NEAR: the near-singular pairs of a policy.
 // Another slot: the pairs of the Galerkin formalism inside that breakpoint of
 // the distance tables that share no node (kept under the mode GAL_LIST + slot).
@@ -617,8 +630,10 @@ void keep_near_list(nb_mesh *trial, const std::shared_ptr<NearList> &nl)
 	c.push_back(nl);
 }
 
+// A list of more than max_pairs pairs is counted and refused: an error for the
+// near-singular pairs, which need theirs, and a list kept as `refused` otherwise.
 int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy pol, hipStream_t st,
-	std::shared_ptr<NearList> *out, int slot = nbk::THR_NEAR)
+	std::shared_ptr<NearList> *out, int slot = nbk::THR_NEAR, long long max_pairs = 0x7fffffff)
 {
 	if (slot != nbk::THR_NEAR) {
 		pol.near_mode = GAL_LIST + slot;
@@ -627,7 +642,7 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 	if ((*out = find_near_list(trial, test, same, pol))) return NB_OK;
 	std::shared_ptr<NearList> nl(new NearList());
 	nl->test_uid = test->uid; nl->test_alive = test->alive; nl->same = same;
-	nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0;
+	nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0; nl->refused = false;
 	if (pol.near_mode != NB_NEAR_NONE) {
 		nbk::ListArgs a;
 		a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = same;
@@ -645,23 +660,32 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 		const size_t ncnt = (size_t)a.n_rows * a.n_chunks;
 		DevPtr counts, offsets, tmp;
 		int s;
-		if ((s = dev_alloc(counts, ncnt * sizeof(int)))) return s;
-		if ((s = dev_alloc(offsets, ncnt * sizeof(int)))) return s;
+		if ((s = dev_alloc(counts, ncnt * sizeof(int) + 16))) return s;
 		a.counts = (int *)counts.get();
-		a.offsets = (const int *)offsets.get();
+		a.total = (unsigned long long *)((char *)counts.get() + (ncnt * sizeof(int) + 7) / 8 * 8);
+		a.offsets = nullptr;
 		a.pi = a.pj = nullptr;
 		const int grid = a.row_tiles * a.n_chunks;
+		launch_zero(a.total, 1, 1, 1, 8, st);
 		hipLaunchKernelGGL(nbk::near_list_kernel<false>, dim3(grid), dim3(256), 0, st, a);
 		NB_HIP(hipGetLastError());
-		size_t tmp_bytes = 0;
-		NB_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, (int *)counts.get(), (int *)offsets.get(), (int)ncnt, st));
-		if ((s = dev_alloc(tmp, tmp_bytes))) return s;
-		NB_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.get(), tmp_bytes, (int *)counts.get(), (int *)offsets.get(), (int)ncnt, st));
-		int last[2];
-		NB_HIP(hipMemcpyAsync(&last[0], (int *)offsets.get() + ncnt - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-		NB_HIP(hipMemcpyAsync(&last[1], (int *)counts.get() + ncnt - 1, sizeof(int), hipMemcpyDeviceToHost, st));
+		unsigned long long total = 0;
+		NB_HIP(hipMemcpyAsync(&total, a.total, sizeof(total), hipMemcpyDeviceToHost, st));
 		NB_HIP(hipStreamSynchronize(st));
-		nl->n = last[0] + last[1];
+		if (total > (unsigned long long)max_pairs) {
+			if (slot == nbk::THR_NEAR) return fail(NB_ERR_RANGE, "too many near-singular pairs");
+			nl->refused = true;
+			keep_near_list(trial, nl);
+			*out = std::move(nl);
+			return NB_OK;
+		}
+		nl->n = (int)total;
+		if ((s = dev_alloc(offsets, ncnt * sizeof(int)))) return s;
+		a.offsets = (const int *)offsets.get();
+		size_t tmp_bytes = 0;
+		NB_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, a.counts, (int *)offsets.get(), (int)ncnt, st));
+		if ((s = dev_alloc(tmp, tmp_bytes))) return s;
+		NB_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.get(), tmp_bytes, a.counts, (int *)offsets.get(), (int)ncnt, st));
 		if ((s = dev_alloc(nl->pi, (size_t)nl->n * sizeof(int)))) return s;
 		if ((s = dev_alloc(nl->pj, (size_t)nl->n * sizeof(int)))) return s;
 		a.pi = (int *)nl->pi.get();
@@ -694,16 +718,15 @@ int gal_chunk(int n_tiles, int sn)
 // gives degree 4 and more (7 points a triangle, 4 x 4 a quadrilateral).  No
 // list (null) when such pairs are many -- over 1/64 of all, beyond the 2^18
 // that a small mesh may have anyway: 64 lanes then share them better than one
-// wave each.
+// wave each -- or when there is no memory for it.
 int ensure_gal_near(nb_mesh *trial, nb_mesh *test, int same, int km, hipStream_t st, std::shared_ptr<NearList> *out)
 {
 	const int slot = km == nbk::SLP ? nbk::THR_1_8 : km == nbk::HSP ? nbk::THR_3_6 : nbk::THR_2_8;
-	out->reset();
-	const double total = (double)test->n * trial->n;
-	if (total >= 2147483648.0) return NB_OK;      // the list's counts are 32-bit
-	int s = ensure_near_list(trial, test, same, nb_policy{}, st, out, slot);
-	if (s) return s;
-	if ((double)(*out)->n * 64.0 > total + 16777216.0) out->reset();
+	const long long most = std::min((long long)test->n * trial->n / 64 + (1ll << 18), 0x7fffffffll);
+	const int s = ensure_near_list(trial, test, same, nb_policy{}, st, out, slot, most);
+	if (s == NB_ERR_OOM) (void)hipGetLastError();
+	else if (s) return s;
+	if (s || (*out)->refused) out->reset();
 	return NB_OK;
 }
 
@@ -837,18 +860,6 @@ int dtype_bytes(int dt)
 	case NB_F64: return 8;
 	default: return 0;
 	}
-}
-
-// zero_kernel over a rows x cols block: one grid row per column (up to 65535,
-// the kernel strides beyond), enough blocks along x for a column of 16-byte words
-void launch_zero(void *out, int64_t ld, int64_t rows, int64_t cols, int elem_bytes, hipStream_t st)
-{
-	if (rows <= 0 || cols <= 0) return;
-	const int64_t words16 = (rows * elem_bytes + 15) / 16;
-	const unsigned gx = (unsigned)std::min<int64_t>((words16 + 255) / 256, 64);
-	const unsigned gy = (unsigned)std::min<int64_t>(cols, 65535);
-	hipLaunchKernelGGL(nbk::zero_kernel, dim3(gx, gy), dim3(256), 0, st, out, (long long)ld, (long long)rows,
-		(long long)cols, elem_bytes);
 }
 
 int check_out(const nb_out *o, int64_t rows, int64_t cols, bool complex_needed)

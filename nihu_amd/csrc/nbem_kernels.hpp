@@ -1691,6 +1691,7 @@ struct ListArgs {
 	int n_rows, n_cols, same_mesh, row_tiles, chunk, n_chunks, tn, sn;
 	const double *tc, *sc, *thr_near;
 	int *counts;            // [n_rows][n_chunks]
+	unsigned long long *total;   // their sum (zero before the count)
 	const int *offsets;     // exclusive scan of counts
 	int *pi, *pj;
 	// element nodes [npe][tn] / [npe][sn]: pairs that share a node are left out (null: none are)
@@ -1742,7 +1743,14 @@ __global__ void __launch_bounds__(256) near_list_kernel(ListArgs a)
 		for (int u = 0; u < 4; ++u) column(j + u, d2[u], lim[u]);
 	}
 	for (; j < j1; ++j) column(j, d2_pair(cix, ciy, ciz, sc[j], sc[a.sn + j], sc[2 * a.sn + j]), thr[j]);
-	if (!FILL) a.counts[(long long)i * a.n_chunks + ch] = cnt;
+	if (!FILL) {
+		a.counts[(long long)i * a.n_chunks + ch] = cnt;
+		// the wave's sum, bit by bit of the lanes' counts (chunk < 2^11)
+		unsigned sum = 0;
+#pragma unroll
+		for (int b = 0; b < 11; ++b) sum += (unsigned)__popcll(__ballot((cnt >> b) & 1)) << b;
+		if ((threadIdx.x & 63) == 0 && sum != 0) atomicAdd(a.total, (unsigned long long)sum);
+	}
 }
 
 struct ClassArgs {

@@ -77,3 +77,40 @@ def test_lists_of_many_test_meshes(nb, form):
     fresh = nb.Mesh(*sphere())
     operator(nb, fresh, fresh, form)
     assert own == fresh.device_bytes()
+
+
+def test_no_memory_for_a_list_that_is_not_taken(nb):
+    # a fine test mesh inside the breakpoints of a few large trial elements: too
+    # many close pairs for a list, and none of them is held
+    from nihu_amd.mesh import cubed_sphere
+    nodes, q = cubed_sphere(64)
+    fine, coarse = nb.Mesh(nodes, q), cubed_sphere(2)
+    used, far = (nb.Mesh(coarse[0] * 1.3 + move, coarse[1]) for move in (0.0, 100.0))
+    for ny in (0, 1):
+        operator(nb, fine, used, "galerkin", ny)
+        operator(nb, fine, far, "galerkin", ny)      # the same tables, no close pair
+        assert used.device_bytes() == far.device_bytes()
+
+
+def test_close_pairs_of_a_large_mesh(nb, orc):
+    # over 2^31 pairs of elements, few of them close: they are listed (the double
+    # layer's call before leaves the list as the only thing that the single
+    # layer's adds), and the rows are the oracle's
+    import torch
+    from nihu_amd.mesh import cubed_sphere
+    nodes, q = cubed_sphere(63)
+    tris = np.ascontiguousarray(np.concatenate([q[:, None, [0, 1, 2]], q[:, None, [0, 2, 3]]], axis=1).reshape(-1, 3))
+    assert len(tris) ** 2 > 2 ** 31
+    m = nb.Mesh(nodes, tris)
+    out = nb.colmajor(m.n_nodes, m.n_nodes, "float32")
+    grown = []
+    for ny in (1, 0):
+        nb.assemble(m, m, out, nb.NB_LAPLACE, 0, ny, accumulate=False, formalism="galerkin_linear")
+        torch.cuda.synchronize()
+        grown.append(m.device_bytes())
+    assert grown[1] > grown[0]
+    rows = np.array([0, 1000, m.n_nodes - 1])
+    el = np.unique(np.nonzero(np.isin(tris, rows))[0]).astype(np.int32)
+    ref = orc.assemble_galerkin(nodes, tris, 0, 0, 0, linear=True, test_elems=el)[rows].real
+    got = out[torch.from_numpy(rows).cuda()].cpu().numpy()
+    assert np.abs(got - ref).max() < 2e-6 * np.abs(ref).max()
