@@ -718,10 +718,21 @@ int gal_chunk(int n_tiles, int sn)
 // gives degree 4 and more (7 points a triangle, 4 x 4 a quadrilateral).  No
 // list (null) when such pairs are many -- over 1/64 of all, beyond the 2^18
 // that a small mesh may have anyway: 64 lanes then share them better than one
-// wave each -- or when there is no memory for it.
+// wave each --, when there is no memory for it, or when the stream is being
+// captured and the list is not there yet: building one waits for the device,
+// which would end the capture.
 int ensure_gal_near(nb_mesh *trial, nb_mesh *test, int same, int km, hipStream_t st, std::shared_ptr<NearList> *out)
 {
 	const int slot = km == nbk::SLP ? nbk::THR_1_8 : km == nbk::HSP ? nbk::THR_3_6 : nbk::THR_2_8;
+	nb_policy key{};
+	key.near_mode = GAL_LIST + slot;
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if (st) (void)hipStreamIsCapturing(st, &capture);
+	if (capture != hipStreamCaptureStatusNone) {
+		*out = find_near_list(trial, test, same, key);
+		if (*out && (*out)->refused) out->reset();
+		return NB_OK;
+	}
 	const long long most = std::min((long long)test->n * trial->n / 64 + (1ll << 18), 0x7fffffffll);
 	const int s = ensure_near_list(trial, test, same, nb_policy{}, st, out, slot, most);
 	if (s == NB_ERR_OOM) (void)hipGetLastError();

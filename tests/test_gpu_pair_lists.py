@@ -114,3 +114,27 @@ def test_close_pairs_of_a_large_mesh(nb, orc):
     ref = orc.assemble_galerkin(nodes, tris, 0, 0, 0, linear=True, test_elems=el)[rows].real
     got = out[torch.from_numpy(rows).cuda()].cpu().numpy()
     assert np.abs(got - ref).max() < 2e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("two", [False, True], ids=["one-mesh", "two-meshes"])
+@pytest.mark.parametrize("quads", [False, True], ids=["triangles", "quadrilaterals"])
+def test_capture_without_a_list(nb, quads, two):
+    # the double layer's call leaves every table that the single layer takes, not
+    # its list: a graph captured then holds the pass that needs none
+    import torch
+    from nihu_amd.mesh import cubed_sphere
+    nodes, el = cubed_sphere(5) if quads else sphere()
+    m = nb.Mesh(nodes, el)
+    t = nb.Mesh(nodes * 1.2, el) if two else m
+    operator(nb, t, m, "galerkin_linear", 1)
+    out = nb.colmajor(t.n_nodes, m.n_nodes)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        nb.assemble(t, m, out, nb.NB_HELMHOLTZ, 0, 0, 3.0, accumulate=False, formalism="galerkin_linear")
+    want = operator(nb, t, m, "galerkin_linear", 0, dtype="complex128")     # with the list
+    for _ in range(3):
+        out.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        # float32 sums in another order: 2^-24 per addition, some 40 to an entry
+        assert (out - want).abs().max() < 2.4e-6 * want.abs().max()
