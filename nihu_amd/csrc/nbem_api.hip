@@ -117,6 +117,7 @@ struct NearList {
 	int same, mode;
 	double limit;
 	int n;
+	bool captured;                    // a graph may hold its addresses: it stays with its meshes
 	bool refused;                     // more pairs than the caller takes as a list: none are held
 	DevPtr pi, pj;
 };
@@ -608,7 +609,8 @@ int near_list_kind(const NearList &nl) { return nl.mode >= GAL_LIST ? 2 : nl.sam
 // Keep a list: those whose test mesh is gone leave, then the least recently
 // used of its kind beyond 8 -- of those against other test meshes beyond 64
 // while they hold less than 256 MB together (a caller that goes round its test
-// meshes, the blocks of a field mesh among them, finds them all again).
+// meshes, the blocks of a field mesh among them, finds them all again).  One
+// that a captured graph may hold does not leave before its meshes.
 void keep_near_list(nb_mesh *trial, const std::shared_ptr<NearList> &nl)
 {
 	auto &c = trial->near_cache;
@@ -619,7 +621,7 @@ void keep_near_list(nb_mesh *trial, const std::shared_ptr<NearList> &nl)
 		if (near_list_kind(*q) == kind && !q->test_alive.expired()) { ++count; bytes += (int64_t)q->n * 8; }
 	for (size_t i = 0; i < c.size();) {
 		const bool gone = c[i]->test_alive.expired();
-		const bool over = near_list_kind(*c[i]) == kind && count > 8 && (kind == 0 || count > 64 || bytes > (256ll << 20));
+		const bool over = !c[i]->captured && near_list_kind(*c[i]) == kind && count > 8 && (kind == 0 || count > 64 || bytes > (256ll << 20));
 		if (!gone && !over) { ++i; continue; }
 		const int64_t b = (int64_t)c[i]->n * 8;
 		if (!gone) { --count; bytes -= b; }
@@ -628,6 +630,14 @@ void keep_near_list(nb_mesh *trial, const std::shared_ptr<NearList> &nl)
 	}
 	trial->bytes += (int64_t)nl->n * 8;
 	c.push_back(nl);
+}
+
+// is the stream being captured into a graph?
+bool capturing(hipStream_t st)
+{
+	hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+	if (st) (void)hipStreamIsCapturing(st, &c);
+	return c != hipStreamCaptureStatusNone;
 }
 
 // A list of more than max_pairs pairs is counted and refused: an error for the
@@ -639,10 +649,13 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 		pol.near_mode = GAL_LIST + slot;
 		pol.near_limit = 0.0;
 	}
-	if ((*out = find_near_list(trial, test, same, pol))) return NB_OK;
+	if ((*out = find_near_list(trial, test, same, pol))) {
+		if (!(*out)->captured && capturing(st)) (*out)->captured = true;
+		return NB_OK;
+	}
 	std::shared_ptr<NearList> nl(new NearList());
 	nl->test_uid = test->uid; nl->test_alive = test->alive; nl->same = same;
-	nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0; nl->refused = false;
+	nl->mode = pol.near_mode; nl->limit = pol.near_limit; nl->n = 0; nl->captured = nl->refused = false;
 	if (pol.near_mode != NB_NEAR_NONE) {
 		nbk::ListArgs a;
 		a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = same;
@@ -726,13 +739,7 @@ int ensure_gal_near(nb_mesh *trial, nb_mesh *test, int same, int km, hipStream_t
 	const int slot = km == nbk::SLP ? nbk::THR_1_8 : km == nbk::HSP ? nbk::THR_3_6 : nbk::THR_2_8;
 	nb_policy key{};
 	key.near_mode = GAL_LIST + slot;
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	if (st) (void)hipStreamIsCapturing(st, &capture);
-	if (capture != hipStreamCaptureStatusNone) {
-		*out = find_near_list(trial, test, same, key);
-		if (*out && (*out)->refused) out->reset();
-		return NB_OK;
-	}
+	if (capturing(st) && !find_near_list(trial, test, same, key)) return NB_OK;
 	const long long most = std::min((long long)test->n * trial->n / 64 + (1ll << 18), 0x7fffffffll);
 	const int s = ensure_near_list(trial, test, same, nb_policy{}, st, out, slot, most);
 	if (s == NB_ERR_OOM) (void)hipGetLastError();

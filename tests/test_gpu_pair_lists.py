@@ -138,3 +138,25 @@ def test_capture_without_a_list(nb, quads, two):
         torch.cuda.synchronize()
         # float32 sums in another order: 2^-24 per addition, some 40 to an entry
         assert (out - want).abs().max() < 2.4e-6 * want.abs().max()
+
+
+def test_a_captured_list_stays(nb):
+    # a graph holds the list's addresses: eighty other test meshes (far away,
+    # their lists are empty) do not displace it
+    import torch
+    m, t = nb.Mesh(*sphere()), nb.Mesh(*sphere(1, 0.3))
+    want = operator(nb, t, m, "galerkin_linear")
+    out = nb.colmajor(t.n_nodes, m.n_nodes)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        nb.assemble(t, m, out, nb.NB_HELMHOLTZ, 0, 0, 3.0, accumulate=False, formalism="galerkin_linear")
+    held = m.device_bytes()
+    others = [nb.Mesh(*sphere(0, 50.0 + i)) for i in range(80)]
+    for o in others:
+        operator(nb, o, m, "galerkin_linear")
+    assert m.device_bytes() == held
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert (out - want).abs().max() < 2.4e-6 * want.abs().max()
