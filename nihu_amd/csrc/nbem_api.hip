@@ -660,7 +660,11 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 		nbk::ListArgs a;
 		a.n_rows = test->n; a.n_cols = trial->n; a.same_mesh = same;
 		a.row_tiles = (test->n + 255) / 256;
+		// short chunks while there are few workgroups (near_list_kernel), but the
+		// counts (4 bytes a row and chunk, as much again for their sums) stay at 64
+		// MB each up to 130000 elements and at 0.1 % of a complex64 matrix beyond
 		a.chunk = 128;
+		while (a.chunk < 1024 && (long long)a.row_tiles * ((trial->n + a.chunk - 1) / a.chunk) > 65536) a.chunk *= 2;
 		a.n_chunks = (trial->n + a.chunk - 1) / a.chunk;
 		a.tn = test->n; a.sn = trial->n;
 		a.tc = (const double *)test->d_c.get();
