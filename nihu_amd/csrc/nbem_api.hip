@@ -33,6 +33,7 @@
 #include <tuple>
 #include <cmath>
 #include <cstdlib>
+#include <cstddef>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -378,9 +379,12 @@ struct nb_mesh {
 	struct GalLayout {
 		int tiles = 0, chunk = 0;
 		DevPtr elem, contrib, rows, fin, first;
+		std::vector<int32_t> order, col;       // host: the sequence, and its slots until the records hold them
 	} glay[2];
-	// Galerkin trial sequences: in the order of glay[0], glay[1], element order
+	// Galerkin trial sequences: in the order of glay[0], glay[1], element order;
+	// the share distances only once a call on one mesh needs them
 	DevPtr d_grec[3];
+	bool grec_share[3] = {false, false, false};
 	DevPtr d_edof;                             // element dof map [npe][n]: e at every corner
 	// Galerkin singular pairs against itself (coincident pairs first)
 	int64_t sp_n = -1;
@@ -802,12 +806,25 @@ int ensure_sing_pairs(nb_mesh *m)
 	return NB_OK;
 }
 
-// The trial sequence records of a mesh (GalRec): order, col as
-// nbg_galerkin_layout_n gives them, or null for element order without slots
-int upload_gal_rec(nb_mesh *m, int kind, const int32_t *order, const int32_t *col)
+// The trial sequence records of a mesh (GalRec), kind 0, 1 in the order and
+// with the slots of glay[kind], 2 in element order without slots; share: with
+// the share distances, which pairs of one mesh are tested by
+int ensure_gal_rec(nb_mesh *m, int kind, bool share)
 {
 	int s;
-	if ((s = ensure_sing_pairs(m))) return s;
+	if (share && (s = ensure_sing_pairs(m))) return s;
+	if (m->d_grec[kind] && (m->grec_share[kind] || !share)) return NB_OK;
+	const int32_t *order = kind < 2 ? m->glay[kind].order.data() : nullptr;
+	if (m->d_grec[kind]) {
+		// in place: nothing that runs without them reads the share distances
+		std::vector<double> v(m->n);
+		for (int i = 0; i < m->n; ++i) v[i] = m->share[order ? order[i] : i];
+		NB_HIP(hipMemcpy2D((char *)m->d_grec[kind].get() + offsetof(nbk::GalRec, share), sizeof(nbk::GalRec), v.data(),
+			sizeof(double), sizeof(double), m->n, hipMemcpyHostToDevice));
+		m->grec_share[kind] = true;
+		return NB_OK;
+	}
+	const int32_t *col = kind < 2 ? m->glay[kind].col.data() : nullptr;
 	const int n = m->n, npe = m->npe;
 	const double four_pi = 4.0 * 3.141592653589793238462643383279502884;
 	// breakpoints of the distance tables of orders 1..3 (ensure_thresholds)
@@ -823,7 +840,7 @@ int upload_gal_rec(nb_mesh *m, int kind, const int32_t *order, const int32_t *co
 			r.near[t] = nbg_threshold(m->R[f], near[t]);
 			r.far[t] = nbg_threshold(m->R[f], far[t]);
 		}
-		r.share = m->share[f];
+		r.share = share ? m->share[f] : 0.0;
 		// one-point weights as in the point tables (the triangles' carry 1 / (4 pi))
 		r.w1 = (float)(npe == 4 ? 4.0 * m->J[f] : 0.5 * m->J[f] / four_pi);
 		for (int c = 0; c < 4; ++c) {
@@ -834,6 +851,8 @@ int upload_gal_rec(nb_mesh *m, int kind, const int32_t *order, const int32_t *co
 		r.elem = f;
 	}
 	if ((s = upload(m->d_grec[kind], rec))) return s;
+	m->grec_share[kind] = share;
+	if (kind < 2) std::vector<int32_t>().swap(m->glay[kind].col);
 	m->bytes += (int64_t)n * sizeof(nbk::GalRec);
 	return NB_OK;
 }
@@ -865,8 +884,10 @@ int ensure_gal_layout(nb_mesh *m, int kind = 0)
 	}
 	int s;
 	if ((s = upload(L.elem, elem)) || (s = upload(L.contrib, contrib)) || (s = upload(L.rows, rows)) ||
-		(s = upload(L.fin, fin)) || (s = upload(L.first, first)) || (s = upload_gal_rec(m, kind, order.data(), col.data())))
+		(s = upload(L.fin, fin)) || (s = upload(L.first, first)))
 		return s;
+	L.order = std::move(order);
+	L.col = std::move(col);
 	L.tiles = tiles;
 	L.chunk = chunk;
 	m->bytes += (int64_t)(elem.size() + rows.size() + contrib.size() + fin.size()) * 4;
@@ -1025,7 +1046,7 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 		if ((s = ensure_gq(trial, N)) || (s = ensure_gq(test, N))) return s;
 	const int kt = lt ? 0 : 1, ks = ls ? 0 : 1;   // layout kinds: node or element dofs
 	if (nodal && ((s = ensure_gal_layout(test, kt)) || (s = ensure_gal_layout(trial, ks)))) return s;
-	if (jb.same && (s = ensure_sing_pairs(trial))) return s;
+	if ((s = ensure_gal_rec(trial, nodal ? ks : 2, jb.same != 0))) return s;
 	std::shared_ptr<NearList> nl;
 	if (fixed_n == 0 && (s = ensure_gal_near(trial, test, jb.same, jb.km, st, &nl))) return s;
 	if (nodal && !accumulate && (s = zero())) return s;
@@ -1043,7 +1064,6 @@ int run_galerkin_quad(const Job &jb, void *out, int64_t ld, int dtype, int accum
 	} else {
 		a.n_tiles = (test->n + nbk::GAL_TILE - 1) / nbk::GAL_TILE;
 		a.chunk = gal_chunk(a.n_tiles, trial->n);
-		if (!trial->d_grec[2] && (s = upload_gal_rec(trial, 2, nullptr, nullptr))) return s;
 		a.rec = (const nbk::GalRec *)trial->d_grec[2].get();
 	}
 	a.tn = test->n; a.sn = trial->n; a.same_mesh = jb.same;
@@ -1217,7 +1237,7 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 		if ((s = ensure_quad(trial, d)) || (s = ensure_quad(test, d))) return s;
 	const int kt = lt ? 0 : 1, ks = ls ? 0 : 1;   // layout kinds: node or element dofs
 	if (nodal && ((s = ensure_gal_layout(test, kt)) || (s = ensure_gal_layout(trial, ks)))) return s;
-	if (jb.same && (s = ensure_sing_pairs(trial))) return s;
+	if ((s = ensure_gal_rec(trial, nodal ? ks : 2, jb.same != 0))) return s;
 	std::shared_ptr<NearList> nl;
 	if (jb.pol.rule != NB_RULE_FIXED && (s = ensure_gal_near(trial, test, jb.same, jb.km, st, &nl))) return s;
 	if (nodal && !accumulate && (s = zero())) return s;
@@ -1239,7 +1259,6 @@ int run_galerkin(const Job &jb, void *out, int64_t ld, int dtype, int accumulate
 	} else {
 		a.n_tiles = (test->n + nbk::GAL_TILE - 1) / nbk::GAL_TILE;
 		a.chunk = gal_chunk(a.n_tiles, trial->n);
-		if (!trial->d_grec[2] && (s = upload_gal_rec(trial, 2, nullptr, nullptr))) return s;
 		a.rec = (const nbk::GalRec *)trial->d_grec[2].get();
 	}
 	// one mesh, one fixed rule, nodal fields on both sides, the single layer: each

@@ -237,3 +237,35 @@ def test_full_size_rows_and_gauss_identity(nb, orc):
     gauss = np.abs(rs_d + 0.5 * ms).max() / ms.max()
     print("Gauss identity max deviation %.2e" % gauss, flush=True)
     assert gauss < 5e-3
+
+
+@pytest.mark.parametrize("form", ["galerkin", "galerkin_linear"])
+@pytest.mark.parametrize("quads", [False, True], ids=["triangles", "quadrilaterals"])
+def test_two_meshes_hold_what_they_need(quads, form):
+    """Between two meshes no pair shares a node: neither mesh holds the singular
+    pairs then (12 bytes each), the test mesh no trial sequence (192 bytes an
+    element); both come with the call that needs them, and what it gives is
+    what it gives on a new mesh."""
+    import torch
+    from nihu_amd import nbem
+    from nihu_amd.mesh import cubed_sphere, jittered_icosphere
+    nodes, el = cubed_sphere(6) if quads else jittered_icosphere(2, seed=3)
+    sets = [set(e) for e in el]
+    n_sing = sum(bool(a & b) for a in sets for b in sets)
+
+    def run(t, m, dtype="complex128"):
+        out = nbem.colmajor(t.dofs(form, "test"), m.dofs(form, "trial"), dtype)
+        nbem.assemble(t, m, out, nbem.NB_HELMHOLTZ, 0, 0, 3.0, accumulate=False, formalism=form)
+        torch.cuda.synchronize()
+        return out
+
+    t, m, fresh = nbem.Mesh(nodes + 40.0, el), nbem.Mesh(nodes, el), nbem.Mesh(nodes, el)
+    run(t, m)
+    before = t.device_bytes(), m.device_bytes()
+    got, want = run(m, m), run(fresh, fresh)
+    # 32-bit sums in varying order where several waves add to an entry
+    assert (got - want).abs().max() < 2.4e-6 * want.abs().max()
+    assert m.device_bytes() - before[1] >= 12 * n_sing
+    run(m, t)
+    assert t.device_bytes() - before[0] >= 192 * t.n
+    assert (run(t, m) - run(nbem.Mesh(nodes + 40.0, el), fresh)).abs().max() < 2.4e-6 * want.abs().max()
