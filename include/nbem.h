@@ -269,6 +269,9 @@ int nb_classify(const nb_mesh *test, const nb_mesh *trial, int32_t same_mesh, in
  * wavenumbers up to 64, quadrature rule).  Fixed rules without a one-launch
  * path return the default shape. */
 int nb_autotune(const nb_mesh *mesh, int32_t n_k, const nb_policy *policy, nb_launch *best);
+/* Launch shape of the single-wavenumber collocation passes of this process:
+ * tile_cols > 0 fixes the trial columns per workgroup, 0 leaves them to the
+ * size of the grid again. */
 int nb_set_launch(const nb_launch *launch);
 
 int nb_synchronize(void *stream);

@@ -3081,6 +3081,8 @@ int nb_set_launch(const nb_launch *launch)
 	if (!launch) return fail(NB_ERR_ARG, "null launch");
 	if (launch->tile_cols < 0 || launch->tile_cols > 4096) return fail(NB_ERR_ARG, "tile_cols out of range");
 	std::lock_guard<std::mutex> lc(g_cfg_mu);
+	// 0 is the default of each: for the columns the rule by the size of the grid
+	g_cfg = LaunchCfg();
 	if (launch->tile_cols) g_cfg.tile_cols = launch->tile_cols;
 	if (launch->k_batch) g_cfg.k_batch = launch->k_batch;
 	if (launch->persistent) g_cfg.persistent = launch->persistent;

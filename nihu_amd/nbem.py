@@ -393,6 +393,8 @@ def autotune(mesh: Mesh, n_k=1, pol=None):
 
 
 def set_launch(tile_cols=0, k_batch=0, persistent=0):
+    """Launch shape of the single-wavenumber collocation passes of this process;
+    0 is the default of each (tile_cols: by the size of the grid)."""
     check(lib().nb_set_launch(C.byref(NbLaunch(tile_cols, k_batch, persistent))))
 
 

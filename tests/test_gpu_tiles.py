@@ -180,3 +180,36 @@ def test_product_sizes(nb, rows, cols, ld):
         ref += (b * x[j:j + 1024]).sum(1)
         mag += (b.abs() * x[j:j + 1024].abs()).sum(1)
     assert ((y - ref).abs() <= cols * 2.0 ** -52 * mag).all()
+
+
+def test_launch_shape_set_and_reset(nb):
+    # a fixed column count serialises a small matrix (5 workgroups of 1280
+    # columns); 0 gives the rule by the grid's size back, and neither changes the
+    # result.  The passes take about 1 ms and 0.02 ms: a factor of 4 is asked for
+    import torch
+    from nihu_amd.mesh import jittered_icosphere
+    nodes, tris = jittered_icosphere(3, seed=0)
+    m = nb.Mesh(nodes, tris)
+
+    def run():
+        A, B = nb.colmajor(m.n, m.n), nb.colmajor(m.n, m.n)
+        nb.assemble_bm(m, 3.0, A, B)
+        nb.profile(True)
+        nb.profile_read(reset=True)
+        for _ in range(5):
+            nb.assemble_bm(m, 3.0, A, B)
+        ms, launches = nb.profile_read(reset=True)["regular"]
+        nb.profile(False)
+        torch.cuda.synchronize()
+        return A, ms / launches
+
+    try:
+        nb.set_launch(tile_cols=4096)
+        fixed, slow = run()
+        nb.set_launch(tile_cols=0)
+        auto, fast = run()
+    finally:
+        nb.set_launch()
+    print("4096 columns %.3f ms, by the grid %.3f ms" % (slow, fast), flush=True)
+    assert torch.equal(torch.view_as_real(fixed), torch.view_as_real(auto))
+    assert fast < slow / 4
