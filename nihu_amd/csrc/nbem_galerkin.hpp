@@ -319,6 +319,15 @@ __device__ __forceinline__ void gal_eval_dynamic(const GalArgs &a, int e, int f,
 	}
 }
 
+// Order between a wave's own LDS accesses from different lanes: the hardware
+// keeps them in program order, and this keeps the compiler from moving one past
+// another that touches no cell of the same lane.  No instruction.
+__device__ __forceinline__ void wave_lds_order()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+	__builtin_amdgcn_wave_barrier();
+}
+
 // Column-slot accumulators in LDS, private to each lane: corner c of slot s at
 // acc[s * SLOT + c * 64 + lane]; the slot's last cell stays zero (the target of
 // unused contributor positions).  NPE corners per element.
@@ -409,14 +418,18 @@ __device__ __forceinline__ void gal_flush(float2 *acc, int lane, int slot, int c
 {
 	float2 *sp = acc + slot * GalSlots<NPE>::SLOT;
 	float2 v[ROWS];
+	wave_lds_order();            // the lanes' adds before the rows' sums
 #pragma unroll
 	for (int r = 0; r < ROWS; ++r) v[r] = row[r].sum(sp, ncon);
+	wave_lds_order();            // which every lane has read before a cell is written over
 #pragma unroll
 	for (int r = 0; r < ROWS; ++r)
 		sp[r * GAL_TILE + lane] = make_float2(a.alpha.x * v[r].x - a.alpha.y * v[r].y, a.alpha.x * v[r].y + a.alpha.y * v[r].x);
 	float part[2 * ROWS];
+	wave_lds_order();
 #pragma unroll
 	for (int t = 0; t < 2 * ROWS; ++t) part[t] = ((const float *)sp)[t * 64 + lane];
+	wave_lds_order();
 	GalSlots<NPE>::clear(acc, lane, slot);
 	const bool real = a.dtype == DT_F32 || a.dtype == DT_F64;
 #pragma unroll
