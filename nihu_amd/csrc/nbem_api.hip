@@ -1976,7 +1976,7 @@ int run_device(const Job &jb, void *out0, void *out1, int64_t ld, int dtype, int
 		else if (mapped) hipLaunchKernelGGL((regular_kernel<F, K, M, Q, true>), dim3(grid), dim3(256), 0, st, a); \
 		else hipLaunchKernelGGL((regular_kernel<F, K, M, Q, false>), dim3(grid), dim3(256), 0, st, a); } while (0)
 		if (jb.mode == OUT_BM) {
-			if (bm_direct(jb)) {
+			if (bm_direct(jb) && a.field_complexity == 0) {
 				if (mapped) hipLaunchKernelGGL((bm_regular_kernel<true>), dim3(grid), dim3(256), 0, st, a);
 				else hipLaunchKernelGGL((bm_regular_kernel<false>), dim3(grid), dim3(256), 0, st, a);
 			} else if (fix7) NB_RG(HELM, ALL4, OUT_BM, 7);

@@ -798,10 +798,9 @@ __device__ __forceinline__ void bm_close(const RegArgs &a, int j, bool act, doub
 	p.d2f = b.d2f; p.df = b.df; p.t0 = b.t0;
 	p.nxx = nxx; p.nxy = nxy; p.nxz = nxz;
 	p.b0 = b.b0;
-	const int fc = a.field_complexity;
 	float2 s[6] = {zero2(), zero2(), zero2(), zero2(), zero2(), zero2()};
-	eval_groups<HELM, ALL4>(a, j, act ? fc + table_degree_rec<1>(d2, t) : -1, act ? fc + table_degree_rec<2>(d2, t) : -1,
-		act ? fc + table_degree_rec<3>(d2, t) : -1, p, w1, b.rinv, b.k, k_revf, s);
+	eval_groups<HELM, ALL4>(a, j, act ? table_degree_rec<1>(d2, t) : -1, act ? table_degree_rec<2>(d2, t) : -1,
+		act ? table_degree_rec<3>(d2, t) : -1, p, w1, b.rinv, b.k, k_revf, s);
 	float2 K[4];
 	kernel_values<HELM, ALL4>(s, b.av, b.nn, b.k, true, K);
 	e.ar = K[1].x - b.ai * K[3].y;
@@ -838,7 +837,9 @@ __device__ __forceinline__ void bm_wave(BmPair &p, double d, double k_rev, float
 }
 
 // Regular pairs of a Burton-Miller assembly under NiHu's distance-driven
-// degrees with an imaginary alpha; organised as regular_kernel.  Three of four
+// degrees with an imaginary alpha; organised as regular_kernel.  Constant
+// fields only: the degrees are the distance tables' own in all three of
+// bm_far, bm_mid and bm_close (field_complexity 0).  Three of four
 // waves take bm_far, most of the others bm_mid, a few per cent bm_close.
 // 20480 triangles: 1.51 ms, 4.4 TB/s of stores; 1.32 ms without the stores,
 // 1.40 ms with the stores alone.
