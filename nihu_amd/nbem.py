@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 
 import numpy as np
 
@@ -160,6 +161,13 @@ def _stream_ptr(stream):
     return C.c_void_p(int(stream))
 
 
+# Blocks that a mesh keeps (Mesh.block): their number -- a surface keeps the near
+# lists of 64 test meshes -- and their elements together, about 200 bytes each on
+# the device.  The lock is re-entrant: a block that leaves is closed under it.
+KEPT_BLOCKS, KEPT_ELEMENTS = 32, 1 << 20
+_BLOCK_LOCK = threading.RLock()
+
+
 class Mesh:
     """A mesh resident on the current GPU (nb_mesh): elements with 3 node
     indices (flat triangles) or 4 (bilinear quadrilaterals); from_elements
@@ -235,26 +243,44 @@ class Mesh:
         return 4 * self.n if f == NB_COLLOCATION_GAUSS else self.n
 
     def device_bytes(self):
+        """device memory of the mesh and of the blocks kept with it"""
         b = C.c_int64()
         check(lib().nb_mesh_info(self._h, None, None, C.byref(b)))
-        return b.value
+        with _BLOCK_LOCK:
+            kept = [e[0] for e in self.__dict__.get("_blocks", {}).values()]
+        return b.value + sum(m.device_bytes() for m in kept)
 
     def block(self, r0, r1, device=0):
-        """The mesh of this mesh's elements r0 .. r1 - 1 on the current device
-        (number `device`: a mesh lives where it was created), kept until this mesh
-        is closed (the latest 32).  A block is built again when the arrays no longer
-        hold what it was built from."""
-        blocks = self.__dict__.setdefault("_blocks", {})
-        sub = blocks.get((device, r0, r1))
-        if sub is None or not (np.array_equal(sub.nodes, self.nodes) and np.array_equal(sub.tris, self.tris[r0:r1])):
-            sub = Mesh(self.nodes.copy(), self.tris[r0:r1].copy())
-            while len(blocks) >= 32:
-                blocks.pop(next(iter(blocks)), None)
-            blocks[(device, r0, r1)] = sub
-        return sub
+        """The mesh of this mesh's elements r0 .. r1 - 1 and their nodes on the
+        current device (number `device`: a mesh lives where it was created), kept
+        until this mesh is closed: the latest used, up to KEPT_BLOCKS of them and
+        KEPT_ELEMENTS elements together.  A block is built again when the arrays no
+        longer hold what it was built from."""
+        key = (device, r0, r1)
+        with _BLOCK_LOCK:
+            blocks = self.__dict__.setdefault("_blocks", {})
+            entry = blocks.pop(key, None)
+            if entry is None or not (np.array_equal(entry[1], self.tris[r0:r1]) and
+                                     np.array_equal(entry[3], self.nodes[entry[2]])):
+                tris = self.tris[r0:r1].copy()
+                if tris.min(initial=0) < 0 or tris.max(initial=0) >= len(self.nodes):
+                    raise ValueError("node index out of range")
+                ids, local = np.unique(tris, return_inverse=True)
+                nodes = self.nodes[ids]
+                entry = (Mesh(nodes, local.reshape(tris.shape)), tris, ids, nodes)
+            size = sum(k[2] - k[1] for k in blocks) + r1 - r0
+            while blocks and (len(blocks) >= KEPT_BLOCKS or size > KEPT_ELEMENTS):
+                old = next(iter(blocks))
+                del blocks[old]
+                size -= old[2] - old[1]
+            if size <= KEPT_ELEMENTS:
+                blocks[key] = entry
+        return entry[0]
 
     def close(self):
-        self.__dict__.pop("_blocks", None)
+        with _BLOCK_LOCK:
+            blocks = self.__dict__.pop("_blocks", None)
+        del blocks
         if getattr(self, "_h", None):
             lib().nb_mesh_destroy(self._h)
             self._h = None

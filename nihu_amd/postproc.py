@@ -47,10 +47,17 @@ def field_pressure(field: "nbem.Mesh", surface: "nbem.Mesh", k: float, p, q, pol
     out = torch.empty(m, dtype=dt, device="cuda")
     # the field mesh's elements in blocks of rows: a sub-mesh per block, kept
     # with the field mesh (building both blocks of 8640 points, their near lists
-    # included, took half of a repeated call's 1.85 ms)
+    # included, took half of a repeated call's 1.85 ms) -- not those of a field
+    # larger than what it keeps, where each would push out the next
+    keep = m <= min(nbem.KEPT_ELEMENTS, block_rows * nbem.KEPT_BLOCKS)
     for r0 in range(0, m, block_rows):
         r1 = min(m, r0 + block_rows)
-        sub = field if (r0 == 0 and r1 == m) else field.block(r0, r1, torch.cuda.current_device())
+        if r0 == 0 and r1 == m:
+            sub = field
+        elif keep:
+            sub = field.block(r0, r1, torch.cuda.current_device())
+        else:
+            sub = nbem.Mesh(field.nodes, field.tris[r0:r1])
         L = nbem.colmajor(r1 - r0, n, dtype)
         M = nbem.colmajor(r1 - r0, n, dtype)
         nbem.assemble(sub, surface, L, nbem.NB_HELMHOLTZ, 0, 0, k, pol=pol, same_mesh=False, accumulate=False)

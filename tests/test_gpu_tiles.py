@@ -162,6 +162,27 @@ def test_field_blocks_follow_the_arrays(nb):
     assert torch.equal(moved, fresh)
 
 
+def test_field_blocks_in_the_byte_count(nb):
+    # the kept blocks are in the field mesh's count; of a field of more blocks
+    # than are kept none stays, and every way of cutting gives the same values
+    import torch
+    from nihu_amd import postproc
+    from nihu_amd.mesh import create_slab
+    nodes, quads = surface(54, quads=True)
+    s = nb.Mesh(nodes, quads)
+    corners = np.array([[-2, -2, 2.5], [2, -2, 2.5], [2, 2, 3], [-2, 2, 3]], dtype=float)
+    field = nb.Mesh(*create_slab(corners, 20, 15))
+    p = torch.ones(54, dtype=torch.complex128, device="cuda")
+    whole = postproc.field_pressure(field, s, 2.0, p, 1j * p)
+    alone = field.device_bytes()
+    many = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=8)      # 38 blocks
+    assert field.device_bytes() == alone
+    few = postproc.field_pressure(field, s, 2.0, p, 1j * p, block_rows=128)
+    assert field.device_bytes() >= 2 * alone - 200
+    for got in (many, few):
+        assert (got - whole).abs().max() <= 1e-12 * whole.abs().max()
+
+
 @pytest.mark.parametrize("rows,cols,ld", [(1, 5, 1), (257, 3001, 300), (8191, 8193, 8191), (8192, 8192, 8192),
                                           (8195, 8195, 8201)])
 def test_product_sizes(nb, rows, cols, ld):
