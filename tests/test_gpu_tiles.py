@@ -139,6 +139,28 @@ def test_galerkin_fixed_single_layer(nb, orc, n_elem, degree, kind):
     assert np.abs(out.cpu().numpy() - old - ref).max() < 2e-6 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("dtype,fam,k,alpha", [("float32", 0, 0.0, 1.0), ("float32", 0, 0.0, -0.75), ("float64", 0, 0.0, 2.5),
+                                               ("complex64", 1, 3.0, 0.8 + 0.25j), ("complex128", 1, 3.0, -0.5j),
+                                               ("complex64", 1, complex(3.0, -0.4), 1.0)])
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("n_elem", [1, 65, 701])
+def test_galerkin_fixed_single_layer_outputs(nb, orc, n_elem, pad, dtype, fam, k, alpha):
+    # the mirrored pairs in every type of result, with rows to spare below each
+    # column (left alone) and a factor; bar as above
+    import torch
+    nodes, el = surface(n_elem)
+    m = nb.Mesh(nodes, el)
+    n = m.n_nodes
+    ref = orc.assemble_galerkin(nodes, el, fam, 0, 0, k=k, alpha=alpha, linear=True, pol=orc.policy(rule=1, fixed_degree=4))
+    full = torch.full((n, n + pad), 7.0, dtype=getattr(torch, dtype), device="cuda")
+    out = full.t()[:n]
+    nb.assemble(m, m, out, fam, 0, 0, k, alpha=alpha, pol=nb.policy("fixed", degree=4), accumulate=False,
+                formalism="galerkin_linear")
+    torch.cuda.synchronize()
+    assert (full[:, n:] == 7.0).all()
+    assert np.abs(out.cpu().numpy() - ref).max() < 2e-6 * np.abs(ref).max()
+
+
 def test_field_blocks_follow_the_arrays(nb):
     # more field points than one block: the kept blocks give the result of a new
     # mesh, also after the field mesh's node array has changed
