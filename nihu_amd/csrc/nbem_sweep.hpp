@@ -79,7 +79,8 @@ __global__ void __launch_bounds__(256) sweep_regular_kernel(SweepArgs a)
 			//   B = sum [W3 - (i/k) W4] e^{-i th}
 			// (seven weights, one per kernel sum, took 14 FMAs per point and
 			// wavenumber instead of 10; 64 wavenumbers on 5120 triangles 10.0 -> 8.3
-			// ms a call)
+			// ms a call.  W3's w / r is taken from the root itself: as r g r it carried
+			// the root's error five times, B's smaller entries 1/3 more error)
 			float gdel[Q], W[5][Q];
 			const auto qf = uni((const float *)(a.qt + (size_t)j * Q));
 #pragma unroll
@@ -91,15 +92,16 @@ __global__ void __launch_bounds__(256) sweep_regular_kernel(SweepArgs a)
 				const float r = r2 * rinv;
 				gdel[q] = u * __builtin_amdgcn_rcpf(r + df);
 				const float ri2 = rinv * rinv;
-				const float g = w * rinv * ri2;
+				const float wr = w * rinv;
+				const float g = wr * ri2;
 				const float b = __builtin_fmaf(oz, nxz, __builtin_fmaf(oy, nxy, __builtin_fmaf(ox, nxx, b0)));
 				const float beta = __builtin_fmaf(-3.0f * av, b * ri2, nn);
 				const float gs = g * (b + r);
 				W[0][q] = g * beta;
 				W[1][q] = g * __builtin_fmaf(beta, r, -av);
 				W[2][q] = av * gs;
-				W[3][q] = r * gs;
 				W[4][q] = g * b;
+				W[3][q] = __builtin_fmaf(W[4][q], r, wr);
 			}
 			for (int fb = 0; fb < KB; ++fb) {
 				const int f = f0 + fb;

@@ -203,3 +203,32 @@ def test_config4_sweep_64_wavenumbers(nb, orc):
         eb = relfro(B[f][ri, :].cpu().numpy(), Br[t])
         print("ka %.2f: A %.2e B %.2e" % (ks[f], ea, eb), flush=True)
         assert ea < 1e-5 and eb < 1e-5
+
+
+def test_sweep_weights_as_precise_as_one_assembly(nb, orc):
+    """A flat surface, where r.n_x = 0 and B is the single layer, k r small: the
+    7-point rule's entries are sums of w / r and their errors those of the
+    weights.  The sweep forms the same w / r from the same root as the
+    single-wavenumber pass, so its errors over the far pairs (some 2e5 entries)
+    have the same size: a tenth more is allowed."""
+    import torch
+    rng = np.random.default_rng(4)
+    n = 16
+    g = np.stack(np.meshgrid(np.arange(n + 1.0), np.arange(n + 1.0), indexing="ij"), axis=-1).reshape(-1, 2)
+    nodes = np.concatenate([(g + rng.uniform(-0.2, 0.2, g.shape)) / n, np.zeros((len(g), 1))], axis=1)
+    q = (np.arange(n)[:, None] * (n + 1) + np.arange(n)).ravel()
+    tris = np.concatenate([np.stack([q, q + n + 1, q + n + 2], 1), np.stack([q, q + n + 2, q + 1], 1)]).astype(np.int32)
+    m = nb.Mesh(nodes, tris)
+    pol = nb.policy(**CONFIG)
+    ks = np.array([0.01, 0.02])
+    A, B = stack(2, m.n), stack(2, m.n)
+    nb.assemble_sweep(m, ks, A, B, pol=pol, launch=nb.NbLaunch(32, 4, 4))
+    for f, k in enumerate(ks):
+        A1, B1 = nb.colmajor(m.n, m.n), nb.colmajor(m.n, m.n)
+        nb.assemble_bm(m, k, A1, B1, pol=pol)
+        torch.cuda.synchronize()
+        ref = orc.assemble_bm(nodes, tris, k, pol=orc.policy(**CONFIG_O))[1]
+        far = orc.classify(nodes, tris, 0, 0, pol=orc.policy(**CONFIG_O)) >= 0
+        err = [np.sqrt(np.mean(np.abs((b.cpu().numpy().real - ref.real)[far] / ref.real[far]) ** 2)) for b in (B[f], B1)]
+        print("k %.2f: rms relative error %.3e in the sweep, %.3e alone, %d pairs" % (k, err[0], err[1], far.sum()), flush=True)
+        assert err[0] < 1.1 * err[1]
