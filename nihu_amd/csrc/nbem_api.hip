@@ -723,9 +723,10 @@ int ensure_near_list(nb_mesh *trial, const nb_mesh *test, int same, nb_policy po
 // trial-sequence chunk per work-group: as long as possible (the slot
 // accumulators flush at every chunk end) while the grid keeps >= 8192
 // work-groups for the 256 CUs, so that the chunks next to a tile's own, whose
-// rules are the largest, do not outlast the rest.  Single and double layer of
-// 9600 quadrilaterals with 2048 / 4096 / 8192 / 16384 work-groups 18.9 / 17.3 /
-// 16.6 / 16.5 ms, of 96 with chunks of at least 64 / 8 elements 1.65 / 0.31 ms.
+// rules are the largest, do not outlast the rest.  Single and double layer with
+// 2048 / 4096 / 8192 / 16384 work-groups: 9600 quadrilaterals 13.5 / 11.6 / 11.0 /
+// 10.7 ms, 20172 triangles 19.0 / 17.9 / 17.4 / 17.3, 4332 1.48 / 1.44 / 1.46 /
+// 1.46; 20480 triangles by one rule 27.6 / 25.8 / 25.5 / 25.3.
 int gal_chunk(int n_tiles, int sn)
 {
 	int ch = 512;
@@ -741,7 +742,13 @@ int gal_chunk(int n_tiles, int sn)
 // that a small mesh may have anyway: 64 lanes then share them better than one
 // wave each --, when there is no memory for it, or when the stream is being
 // captured and the list is not there yet: building one waits for the device,
-// which would end the capture.
+// which would end the capture.  Of 98304 triangles against 432 to 15552 large
+// ones, with the list / without it: 6.9 % of the pairs close 0.81 / 0.48 ms, 2.4 %
+// 0.95 / 0.76, 0.9 % 1.18 / 1.45, 0.4 % 1.63 / 2.46 (constant fields; nodal 2.4 %
+// 2.29 / 1.73, 0.35 % 6.29 / 5.74, 0.12 % 13.6 / 13.7, double layer 0.95 % 8.43 /
+// 8.40, 0.38 % 15.3 / 15.9); quadrilaterals gain at any share (24576 against 216,
+// 12.8 % 0.54 / 1.32).  A sphere of 4332 triangles has 0.3 % (single layer) and
+// 1.3 % (double layer).
 int ensure_gal_near(nb_mesh *trial, nb_mesh *test, int same, int km, hipStream_t st, std::shared_ptr<NearList> *out)
 {
 	const int slot = km == nbk::SLP ? nbk::THR_1_8 : km == nbk::HSP ? nbk::THR_3_6 : nbk::THR_2_8;

@@ -420,8 +420,10 @@ __device__ __forceinline__ void accumulate_centroid(const PairCtx &p, float w1, 
 // offsets s1 D_m and s2 D_m; table order: centre, s1 (D_2, D_0, D_1), s2 (D_2, D_0,
 // D_1).  Per pair two products dc.D_m and two n_x.D_m give u and b of the six outer
 // points in one FMA each (three for a general point), and the centre needs neither
-// a root nor a reciprocal: about 245 VALU instructions a pair instead of 269 and
-// two transcendentals fewer (20480 triangles, regular pass 3.10 -> 2.95 ms).
+// a root nor a reciprocal: the regular pass takes 272.9 VALU instructions a pair
+// instead of 296.7 (counted, prologue included) and two transcendentals fewer,
+// 3.10 -> 2.92 ms on 20480 triangles.  At one instruction every 3.94 cycles per
+// SIMD it is at the issue limit.
 template <int FAM, int MASK, bool CK = false>
 __device__ __forceinline__ void accumulate_seven(const QPoint *qp_in, const PairCtx &p, float rinv_d, float k_revf, float k,
 	float2 (&s)[6], float ki = 0.0f)
